@@ -202,9 +202,8 @@ int onpu_moe_status(void * h);
 /* ---- weight codecs on the GPU (load time). The reference quantizes on the host (onpu_pack,
  * onpu_api.cpp:499-504, with the search quantizers of opennpu_core.hpp:103-169) and transcodes GGUF
  * Q4_K for its ggml backend on the host (ggml-opennpu.cpp:103-138); these run the same codecs on
- * weights already in HBM and write the handle's tiled layout directly. They allocate a temporary
- * staging buffer (at most 256 MiB, or one expert) and return after their launches on `stream`
- * completed; calls on one handle are serialised by the library mutex. 0 ok, -1 error
+ * weights already in HBM and write the handle's tiled layout directly. They allocate nothing and
+ * return after their launches on `stream` completed (so not under capture); calls on one handle are serialised by the library mutex. 0 ok, -1 error
  * (onpu_last_error). */
 /* experts [e0, e0 + n) of a dense (E = 1) or bank handle from W [n][N][ldw] (row stride ldw >= K
  * elements), fp32 (w_bf16 = 0) or bf16 (1), with the handle's format: the codes and parameters

@@ -1680,28 +1680,22 @@ int64_t onpu_pack_q4k(const uint8_t * blocks, int64_t N, int64_t K, uint8_t * ou
 }  // extern "C"
 
 // ---------------------------------------------------------------- GPU weight codecs
-// Experts [e0, e0 + n) of m from a device source: fill(e, k, staging, stride) writes the staging of
-// experts e .. e + k - 1 (stride bytes apart) on stream s, which is then repacked into the tiled
-// layout. The staging is a temporary of at most 256 MiB (or one expert), freed before returning,
-// so the call waits for its launches.
+// Experts [e0, e0 + n) of m from a device source: fill(e, k, tiles) writes the tiled weights of experts
+// e .. e + k - 1 on stream s, at most 65535 per launch. The call waits for its launches, so it is
+// refused under capture.
 template <class Fill>
 static int codec_load(Mat4 * m, int64_t e0, int64_t n, hipStream_t s, Fill fill) {
-    const int64_t sb = round_up(stage_bytes(m->fmt, m->N, m->K), 256);
-    const int64_t chunk = std::max<int64_t>(1, std::min<int64_t>(n, ((int64_t) 256 << 20) / sb));
     if (n == 0) return 0;
-    void * tmp = nullptr;
-    HIPR(hipMalloc(&tmp, (size_t) (chunk * sb)));
+    hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
+    HIPR(hipStreamIsCapturing(s, &cap));
+    if (cap != hipStreamCaptureStatusNone) { set_err("weight codec: the stream is capturing"); return -1; }
     hipError_t e = hipSuccess;
-    for (int64_t c = 0; c < n && e == hipSuccess; c += chunk) {
-        const int64_t k = std::min(chunk, n - c);
-        e = fill(e0 + c, k, (uint8_t *) tmp, sb);
-        if (e == hipSuccess)
-            e = launch_repack(m->fmt, (const uint8_t *) tmp, sb, m->N, m->K, m->dev + (e0 + c) * m->dstride, m->dstride,
-                              k, s);
+    for (int64_t c = 0; c < n && e == hipSuccess; c += 65535) {
+        const int64_t k = std::min<int64_t>(65535, n - c);
+        e = fill(e0 + c, k, m->dev + (e0 + c) * m->dstride);
         if (e == hipSuccess) e = refresh_dec(m, e0 + c, k, s);
     }
     const hipError_t es = hipStreamSynchronize(s);
-    (void) hipFree(tmp);
     if (e == hipSuccess) e = es;
     if (e != hipSuccess) { set_err("weight codec", e); return -1; }
     return 0;
@@ -1718,8 +1712,8 @@ int onpu_quantize_dev(void * h, int64_t e0, int64_t n, const void * W, int64_t l
     std::lock_guard<std::mutex> lk(g_mu);
     const hipStream_t s = (hipStream_t) stream;
     const int64_t es = m->N * ldw * (w_bf16 ? 2 : 4);           // bytes per expert of W
-    return codec_load(m, e0, n, s, [&](int64_t e, int64_t k, uint8_t * st, int64_t sb) {
-        return launch_quant_stage(m->fmt, (const char *) W + (e - e0) * es, ldw, w_bf16, m->N, m->K, k, st, sb, s);
+    return codec_load(m, e0, n, s, [&](int64_t e, int64_t k, uint8_t * tiles) {
+        return launch_quantize(m->fmt, (const char *) W + (e - e0) * es, ldw, w_bf16, m->N, m->K, k, tiles, m->dstride, s);
     });
 }
 
@@ -1787,8 +1781,8 @@ int onpu_transcode_q4k_dev(void * h, int64_t e0, int64_t n, const void * blocks,
     std::lock_guard<std::mutex> lk(g_mu);
     const hipStream_t s = (hipStream_t) stream;
     const int64_t es = m->N * ld;                                 // bytes per expert of the blocks
-    return codec_load(m, e0, n, s, [&](int64_t e, int64_t k, uint8_t * st, int64_t sb) {
-        return launch_q4k_stage((const uint8_t *) blocks + (e - e0) * es, ld, es, m->N, m->K, k, st, sb, s);
+    return codec_load(m, e0, n, s, [&](int64_t e, int64_t k, uint8_t * tiles) {
+        return launch_q4k((const uint8_t *) blocks + (e - e0) * es, ld, es, m->N, m->K, k, tiles, m->dstride, s);
     });
 }
 

@@ -167,34 +167,41 @@ ONPU_HD uint16_t bf16_step(uint16_t h, int dir) {
 // keeps exactly; its scale d sc and min -dmin mn become the bf16 pair, among the 3 x 3 neighbours
 // of their rounded values, with the least squared error against the exact weights (first minimum
 // in the order scale step -1, 0, 1 outer, min step inner).
-ONPU_HD void q4k_sub(const uint8_t * b, int sub, uint8_t (&q)[32], uint16_t & s_out, uint16_t & m_out) {
+// h: the super-block's first 16 bytes, c: the 32 bytes with the sub-block's nibbles (little-endian dwords).
+ONPU_HD void q4k_sub(const uint32_t (&h)[4], const uint32_t (&c)[8], int sub, uint8_t (&q)[32], uint16_t & s_out,
+                     uint16_t & m_out) {
 #pragma clang fp contract(off)
-    const float d = f16_to_f32((uint16_t) (b[0] | (b[1] << 8))), dmin = f16_to_f32((uint16_t) (b[2] | (b[3] << 8)));
-    const uint8_t * sc = b + 4, * qs = b + 16;
-    uint32_t sv, mv;
-    if (sub < 4) {
-        sv = sc[sub] & 63u;
-        mv = sc[sub + 4] & 63u;
-    } else {
-        sv = (sc[sub + 4] & 0xFu) | ((uint32_t) (sc[sub - 4] >> 6) << 4);
-        mv = (uint32_t) (sc[sub + 4] >> 4) | ((uint32_t) (sc[sub] >> 6) << 4);
-    }
-    const uint8_t * qq = qs + (sub / 2) * 32;
-#pragma unroll
-    for (int l = 0; l < 32; l++) q[l] = (sub & 1) ? (uint8_t) (qq[l] >> 4) : (uint8_t) (qq[l] & 0xF);
+    const float d = f16_to_f32((uint16_t) (h[0] & 0xffffu)), dmin = f16_to_f32((uint16_t) (h[0] >> 16));
+    const int sh = 8 * (sub & 3);
+    const uint32_t b0 = (h[1] >> sh) & 0xffu, b1 = (h[2] >> sh) & 0xffu, b2 = (h[3] >> sh) & 0xffu;
+    const uint32_t sv = sub < 4 ? b0 & 63u : (b2 & 0xFu) | ((b0 >> 6) << 4);
+    const uint32_t mv = sub < 4 ? b1 & 63u : (b2 >> 4) | ((b1 >> 6) << 4);
     const float S = d * (float) sv, M = -dmin * (float) mv;
     const uint16_t s0 = f32_to_bf16(S), m0 = f32_to_bf16(M);
+    float qf[32], w[32];                                                 // codes and exact weights
+#pragma unroll
+    for (int l = 0; l < 32; l++) {
+        q[l] = (uint8_t) ((c[l / 4] >> (8 * (l % 4) + 4 * (sub & 1))) & 0xFu);
+        qf[l] = (float) q[l];
+        w[l] = qf[l] * S + M;
+    }
     float best = __builtin_inff();
     s_out = s0;
     m_out = m0;
+#pragma nounroll
     for (int ds = -1; ds <= 1; ds++)
+#pragma nounroll
         for (int dm = -1; dm <= 1; dm++) {
             const uint16_t sc_ = ds ? bf16_step(s0, ds) : s0, mn_ = dm ? bf16_step(m0, dm) : m0;
             const float sf = bf16_to_f32(sc_), mf = bf16_to_f32(mn_);
             float e = 0;
 #pragma unroll
             for (int l = 0; l < 32; l++) {
-                const float t = q[l] * sf + mf - (q[l] * S + M);
+#ifdef __HIP_DEVICE_COMPILE__
+                const float t = __builtin_fmaf(qf[l], sf, mf) - w[l];    // 4-bit times 8-bit: an exact product
+#else
+                const float t = qf[l] * sf + mf - w[l];
+#endif
                 e += t * t;
             }
             if (e < best) { best = e; s_out = sc_; m_out = mn_; }

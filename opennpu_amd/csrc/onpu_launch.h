@@ -246,13 +246,13 @@ hipError_t argmax_scratch_init();
 hipError_t argmax_scratch_get(int64_t rows, int64_t N, uint64_t ** keys, uint32_t ** cnt);
 hipError_t launch_argmax(const float * v, int64_t rows, int64_t N, int32_t * out, uint64_t * keys, uint32_t * cnt,
                          hipStream_t s);
-// GPU weight codecs (onpu_codec.hip): W [ne][N][ldw] fp32 (wbf16 = 0) or bf16 -> ne staging buffers of
-// format fmt, ostride bytes apart (a multiple of 16); Q4_K rows (ld bytes apart, experts bstride
-// bytes apart) -> q4nx staging
-hipError_t launch_quant_stage(int fmt, const void * W, int64_t ldw, int wbf16, int64_t N, int64_t K, int64_t ne,
-                              uint8_t * out, int64_t ostride, hipStream_t s);
-hipError_t launch_q4k_stage(const uint8_t * blocks, int64_t ld, int64_t bstride, int64_t N, int64_t K, int64_t ne,
-                            uint8_t * out, int64_t ostride, hipStream_t s);
+// GPU weight codecs (onpu_codec.hip): W [ne][N][ldw] fp32 (wbf16 = 0) or bf16 -> ne matrices in the tiled
+// layout of format fmt, ostride bytes apart; Q4_K rows (ld bytes apart, experts bstride bytes apart)
+// -> q4nx tiles
+hipError_t launch_quantize(int fmt, const void * W, int64_t ldw, int wbf16, int64_t N, int64_t K, int64_t ne,
+                           uint8_t * out, int64_t ostride, hipStream_t s);
+hipError_t launch_q4k(const uint8_t * blocks, int64_t ld, int64_t bstride, int64_t N, int64_t K, int64_t ne,
+                      uint8_t * out, int64_t ostride, hipStream_t s);
 // int8 GEMV y = s * (W x) for int8 W [N][K] rows (K a multiple of 16, K * 4 bytes of x in LDS)
 hipError_t launch_gemv_i8(const int8_t * W, const float * sc, int64_t N, int64_t K, const float * x, float * y,
                           hipStream_t s);

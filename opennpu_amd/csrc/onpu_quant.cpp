@@ -90,7 +90,11 @@ static void q4k_rows(const uint8_t * blocks, int64_t ld, int64_t N, int64_t K, i
     for (int64_t r = r0; r < r1; r++)
         for (int64_t g = 0; g < K / 32; g++) {
             uint16_t s = 0, m = 0;
-            q4k_sub(blocks + r * ld + (g / 8) * Q4K_BLOCK, (int) (g % 8), q, s, m);
+            const uint8_t * b = blocks + r * ld + (g / 8) * Q4K_BLOCK;
+            uint32_t h[4], c[8];
+            std::memcpy(h, b, sizeof(h));
+            std::memcpy(c, b + 16 + (g % 8) / 2 * 32, sizeof(c));
+            q4k_sub(h, c, (int) (g % 8), q, s, m);
             for (int i = 0; i < 32; i += 2) out[r * (K / 2) + (32 * g + i) / 2] = (uint8_t) (q[i] | (q[i + 1] << 4));
             sc[r * (K / 32) + g] = s;
             mn[r * (K / 32) + g] = m;

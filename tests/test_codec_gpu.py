@@ -55,6 +55,45 @@ def test_quantize_dev_equals_oracle(gpu, fmt, wdt):
         assert np.array_equal(got.view(np.uint32), want.view(np.uint32)), (fmt, wdt, N, K)
 
 
+def _structured(rng, kind, N, K):
+    """rows whose quotients x / d sit on and next to half-integers, and rows out of the range the
+    division-free search covers (its waves then take the general one)"""
+    if kind == "ties":                              # few mantissa bits: exact ties in both passes
+        W = rng.integers(-40, 41, (N, K)) * (1 + rng.integers(0, 128, (N, 1)) / 128)
+    elif kind == "grid":                            # maxima 9, 8, 13 / 2, ... times a power of two
+        W = rng.integers(-18, 19, (N, K)) * 2.0 ** rng.integers(-12, 3, (N, 1))
+    elif kind == "offset":                          # a min far larger than the scale
+        W = 1000 + rng.standard_normal((N, K)) * 2.0 ** rng.integers(-12, 8, (N, 1))
+    else:                                           # "range": row scales 2^-100 to 2^60, some zero groups
+        W = rng.standard_normal((N, K)) * 2.0 ** rng.integers(-100, 60, (N, 1))
+        W[:, 32:64] = 0
+    return W.astype(np.float32)
+
+
+@pytest.mark.parametrize("kind", ["ties", "grid", "offset", "range"])
+@pytest.mark.parametrize("wdt", ["f32", "bf16"])
+@pytest.mark.parametrize("fmt", [orc.FMT_Q4NX, orc.FMT_Q4S, orc.FMT_G128S])
+def test_quantize_dev_at_ties_and_range_ends(gpu, fmt, wdt, kind):
+    """the search quantizers' quotients by reciprocal, bit for bit the oracle's codes and parameters,
+    with ragged row tiles (a wave's lanes past the matrix) and, per 32, a ragged last block"""
+    import torch
+    from opennpu_amd.device import QMatrix
+    N, K = 149, 640 if fmt == orc.FMT_G128S else 672
+    W = _structured(np.random.default_rng(80 + fmt), kind, N, K)
+    Wd = torch.from_numpy(W)
+    if wdt == "bf16":
+        W = _bf16_round(W)
+        Wd = torch.from_numpy(orc.f2bf_np(W).view(np.int16)).view(torch.bfloat16)
+    q = QMatrix(N, K, fmt)
+    try:
+        q.quantize(Wd.cuda())
+        got = q.dequant()
+    finally:
+        q.free()
+    want = orc.dequant(fmt, orc.quantize(fmt, W), N, K)
+    assert np.array_equal(got.view(np.uint32), want.view(np.uint32))
+
+
 def test_quantize_dev_strided_rows_and_gemv(gpu):
     """rows ldw > K apart (a column slice of a wider tensor); the quantized matrix's GEMV equals
     that of the same matrix loaded from the oracle's staging bytes, bit for bit"""
