@@ -214,97 +214,77 @@ __global__ __launch_bounds__(AKEY_THREADS) void k_argmax_keys(const uint64_t * _
 
 // ------------------------------------------------------------------ int8 GEMV
 // y[n] = s[n] * sum_k W[n][k] x[k] for int8 W [N][K] (the reference's host onpu_gemv_i8,
-// onpu_cpu.cpp:276-299, for a MoE's shared expert). Rows go in groups of 4; a group's K range is
-// split into ks slices (4 below 8192 groups, then 2, then 1), one wave per (group,
-// slice), 4 / ks groups per workgroup. In a wave a row is read by 16 consecutive lanes, 16 bytes
-// each (a wave instruction covers the 4 rows, 1 KiB), GI8_U loads per lane in flight per batch.
-// x sits in LDS (copied once per workgroup with its sum); the four rows' lanes read the same x (a
-// broadcast). The bytes are biased to u = w + 128 by one xor per dword and converted by
-// v_cvt_f32_ubyteN, so a weight costs a convert and an fma, and 128 sum(x) is subtracted once.
-// The 16 lanes of a row sum by DPP, the slices in LDS.
-constexpr int GI8_T = 256, GI8_U = 8;
-
+// onpu_cpu.cpp:276-299, for a MoE's shared expert). A wave takes 4 rows and one of ks K slices; its
+// lane l takes the dwords (4 weights) at k = 4 l + 256 u, u < U per batch, so that the x of those
+// weights is one float4 per step, 16 bytes a lane, and stays in registers for the 4 rows: x and W
+// loads all go out together and one memory latency covers a batch. Bound by that latency and, for
+// large matrices, by HBM. (x in LDS, staged before the first W load and read back at 64-byte strides
+// for every 16 weights of a row, was the bound before: 11264 x 2048 took 14.5 us a call and now
+// 7.3, the rate at which a caller issues them; 16384 x 4096 33.5 -> 17.1 us, 16384 x 16384 140 -> 56.6 us,
+// 4.7 TB/s.) A weight costs one signed byte conversion and one fma; the biased bytes it took before
+// also cost accuracy (error against 64 bits 8.5e-7 -> 1.3e-7).
+constexpr int GI8_R = 4;                     // rows per wave
 template <int CTRL> DEV float dpp_fl(float v) {
     return __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), CTRL, 0xf, 0xf, false));
 }
 
-__global__ __launch_bounds__(GI8_T) void k_gemv_i8(const int8_t * __restrict__ W, const float * __restrict__ s,
-                                                   int64_t N, int64_t K, int ks, int64_t Kw,
-                                                   const float * __restrict__ x, float * __restrict__ y) {
-    extern __shared__ __align__(16) float xs[];
-    __shared__ float wsx[GI8_T / 64];
-    __shared__ float red[GI8_T / 64][4];
-    const int t = threadIdx.x, lane = t & 63, wave = t >> 6, li = lane & 15, slot = lane >> 4;
-    // x to LDS: all of a thread's loads of a batch issued before the stores (8 x 1024 floats per
-    // batch). Buffer loads over x's K floats (the host keeps K * 4 < 2^31): past K they return
-    // zeros, so the loads need no branch (a load under a branch is waited for where the branch
-    // rejoins, which would serialize the batch).
-    float part = 0.f;
-    const __amdgpu_buffer_rsrc_t xr = __builtin_amdgcn_make_buffer_rsrc((void *) x, (short) 0, (int) (K * 4), 0x00020000);
-    for (int64_t k0 = 4 * t; k0 < K; k0 += 8 * 4 * GI8_T) {
-        float4 v[8];
+// grid (row groups / (waves per workgroup / ks)); waves of a row group are consecutive in a workgroup
+template <int U>
+__global__ __launch_bounds__(1024) void k_gemv_i8(const int8_t * __restrict__ W, const float * __restrict__ s,
+                                                  int64_t N, int K, int lks, int Kw, const float * __restrict__ x,
+                                                  float * __restrict__ y) {
+    __shared__ float red[16][GI8_R];
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), ks = 1 << lks, gl = wave >> lks;
+    const int64_t row0 = ((int64_t) blockIdx.x * (blockDim.x >> (6 + lks)) + gl) * GI8_R;
+    const int nr = N - row0 >= GI8_R ? GI8_R : (N > row0 ? (int) (N - row0) : 0);
+    const int k0 = (wave - gl * ks) * Kw, k1 = k0 + Kw < K ? k0 + Kw : K;
+    // Buffer loads without branches: x past the slice reads as zero, W past the rows too (and past the
+    // slice inside them bytes that meet those zeros)
+    const __amdgpu_buffer_rsrc_t xr = __builtin_amdgcn_make_buffer_rsrc((void *) x, (short) 0, k1 * 4, 0x00020000);
+    const __amdgpu_buffer_rsrc_t wr =
+        __builtin_amdgcn_make_buffer_rsrc((void *) (W + (nr ? row0 : 0) * K), (short) 0, nr * K, 0x00020000);
+    float acc[GI8_R] = {};
+    for (int kb = k0; kb < k1; kb += 256 * U) {
+        uint32_t w[GI8_R][U];
+        float4 xv[U];
 #pragma unroll
-        for (int i = 0; i < 8; i++) {
-            const int64_t k = k0 + (int64_t) i * 4 * GI8_T;
-            v[i] = __builtin_bit_cast(float4, __builtin_amdgcn_raw_buffer_load_b128(xr, (uint32_t) (k * 4), 0, 0));
-        }
+        for (int u = 0; u < U; u++)
+            xv[u] = __builtin_bit_cast(float4, __builtin_amdgcn_raw_buffer_load_b128(xr, (uint32_t) (16 * lane), 4 * (kb + 256 * u), 0));
 #pragma unroll
-        for (int i = 0; i < 8; i++) {
-            const int64_t k = k0 + (int64_t) i * 4 * GI8_T;
-            if (k < K) *(float4 *) (xs + k) = v[i];
-            part += (v[i].x + v[i].y) + (v[i].z + v[i].w);
-        }
-    }
-    for (int o = 32; o > 0; o >>= 1) part += __shfl_xor(part, o);
-    if (lane == 0) wsx[wave] = part;
-    __syncthreads();
-    const float xsum = (wsx[0] + wsx[1]) + (wsx[2] + wsx[3]);
-    const int gpw = 4 / ks;
-    const int64_t grp = (int64_t) blockIdx.x * gpw + wave / ks, row = grp * 4 + slot;
-    const int64_t k0 = (wave % ks) * Kw, k1 = k0 + Kw < K ? k0 + Kw : K;
-    const int8_t * wr = W + (row < N ? row : 0) * K;
-    float acc = 0.f;
-    // all GI8_U loads of a step unconditional: past k1 a lane re-reads its own first 16 bytes of
-    // the step (never used: the products below stop at k1)
-    for (int64_t kb = k0 + 16 * li; kb < k1; kb += 256 * GI8_U) {
-        uint4 q[GI8_U];
+        for (int r = 0; r < GI8_R; r++)
 #pragma unroll
-        for (int u = 0; u < GI8_U; u++) {
-            const int64_t k = kb + 256 * u;
-            q[u] = *(const uint4 *) (wr + (k < k1 ? k : kb));
-        }
+            for (int u = 0; u < U; u++)
+                w[r][u] = __builtin_amdgcn_raw_buffer_load_b32(wr, (uint32_t) (4 * lane), r * K + kb + 256 * u, 0);
 #pragma unroll
-        for (int u = 0; u < GI8_U; u++) {
-            const int64_t k = kb + 256 * u;
-            if (k >= k1) break;
-            const uint32_t d[4] = {q[u].x ^ 0x80808080u, q[u].y ^ 0x80808080u, q[u].z ^ 0x80808080u,
-                                   q[u].w ^ 0x80808080u};
+        for (int r = 0; r < GI8_R; r++)
 #pragma unroll
-            for (int i = 0; i < 4; i++) {
-                const float4 xv = *(const float4 *) (xs + k + 4 * i);
-                acc += (float) (d[i] & 0xffu) * xv.x;
-                acc += (float) ((d[i] >> 8) & 0xffu) * xv.y;
-                acc += (float) ((d[i] >> 16) & 0xffu) * xv.z;
-                acc += (float) (d[i] >> 24) * xv.w;
+            for (int u = 0; u < U; u++) {
+                acc[r] += (float) (int8_t) w[r][u] * xv[u].x;
+                acc[r] += (float) (int8_t) (w[r][u] >> 8) * xv[u].y;
+                acc[r] += (float) (int8_t) (w[r][u] >> 16) * xv[u].z;
+                acc[r] += (float) (int8_t) (w[r][u] >> 24) * xv[u].w;
             }
-        }
     }
-    acc += dpp_fl<0xB1>(acc);               // quad_perm [1, 0, 3, 2]
-    acc += dpp_fl<0x4E>(acc);               // quad_perm [2, 3, 0, 1]
-    acc += dpp_fl<0x141>(acc);              // row_half_mirror
-    acc += dpp_fl<0x140>(acc);              // row_mirror
+#pragma unroll
+    for (int r = 0; r < GI8_R; r++) {
+        acc[r] += dpp_fl<0xB1>(acc[r]);      // quad_perm [1, 0, 3, 2]
+        acc[r] += dpp_fl<0x4E>(acc[r]);      // quad_perm [2, 3, 0, 1]
+        acc[r] += dpp_fl<0x141>(acc[r]);     // row_half_mirror
+        acc[r] += dpp_fl<0x140>(acc[r]);     // row_mirror
+        acc[r] += __shfl_xor(acc[r], 16);
+        acc[r] += __shfl_xor(acc[r], 32);
+    }
+    const float v = lane == 0 ? acc[0] : (lane == 1 ? acc[1] : (lane == 2 ? acc[2] : acc[3]));
     if (ks == 1) {
-        if (li == 0 && row < N) y[row] = (acc - 128.0f * xsum) * s[row];
+        if (lane < nr) y[row0 + lane] = v * s[row0 + lane];
         return;
     }
-    if (li == 0) red[wave][slot] = acc;
+    if (lane < GI8_R) red[wave][lane] = v;
     __syncthreads();
-    if (t < 4 * gpw) {
-        const int gl = t / 4;
-        const int64_t r = ((int64_t) blockIdx.x * gpw + gl) * 4 + (t & 3);
+    if (wave == gl * ks && lane < nr) {
         float sum = 0.f;
-        for (int sl = 0; sl < ks; sl++) sum += red[gl * ks + sl][t & 3];
-        if (r < N) y[r] = (sum - 128.0f * xsum) * s[r];
+        for (int i = 0; i < ks; i++) sum += red[wave + i][lane];
+        y[row0 + lane] = sum * s[row0 + lane];
     }
 }
 
@@ -800,15 +780,21 @@ hipError_t launch_gemv_i8(const int8_t * W, const float * sc, int64_t N, int64_t
                           hipStream_t s) {
     if (N <= 0 || K <= 0) return hipSuccess;
     if (K % 16 || K * 4 > 128 * 1024 || ((uintptr_t) W | (uintptr_t) x) % 16) return hipErrorInvalidValue;
-    const int64_t ng = (N + 3) / 4;
-    // K parts per row: more, shorter waves win, except that a row of one full step (256 GI8_U
-    // bytes) stays whole (11264 x 2048: 15.1 us against 15.9 with 4 parts; 2048 x 5632 keeps 4
-    // parts: 8.8 us against 9.4 with 2)
-    const int ks = K <= 256 * GI8_U ? 1 : (ng >= 16384 ? 1 : (ng >= 8192 ? 2 : 4));
+    const int64_t ng = (N + GI8_R - 1) / GI8_R;
+    // K slices until there are 8 waves per CU or a slice is 1024 long (one batch of 4 loads per row):
+    // with few rows the waves in flight are what brings the bytes in (512 x 16384, 16 slices: 11.5 ->
+    // 7.5 us, 2048 x 5632, 4 slices: 8.5 -> 7.4; from 2048 groups one wave per group is enough)
+    int lks = 0;
+    while (lks < 4 && (ng << lks) < 2048 && K > ((int64_t) 1024 << lks)) lks++;
+    const int ks = 1 << lks;
     const int64_t Kw = (K + (int64_t) ks * 256 - 1) / ((int64_t) ks * 256) * 256;
-    const int64_t grid = (ng + 4 / ks - 1) / (4 / ks);
-    if (grid >= ((int64_t) 1 << 31) || K * 4 >= ((int64_t) 1 << 31)) return hipErrorInvalidValue;
-    k_gemv_i8<<<(unsigned) grid, GI8_T, (size_t) K * 4, s>>>(W, sc, N, K, ks, Kw, x, y);
+    const int waves = ks > 4 ? ks : 4;
+    const int64_t grid = (ng + waves / ks - 1) / (waves / ks);
+    if (grid >= ((int64_t) 1 << 31)) return hipErrorInvalidValue;
+    const dim3 g((unsigned) grid), t((unsigned) (64 * waves));
+    if (Kw <= 512) k_gemv_i8<2><<<g, t, 0, s>>>(W, sc, N, (int) K, lks, (int) Kw, x, y);
+    else if (Kw <= 1024) k_gemv_i8<4><<<g, t, 0, s>>>(W, sc, N, (int) K, lks, (int) Kw, x, y);
+    else k_gemv_i8<8><<<g, t, 0, s>>>(W, sc, N, (int) K, lks, (int) Kw, x, y);
     CHECK_LAUNCH();
     return hipSuccess;
 }

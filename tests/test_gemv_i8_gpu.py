@@ -11,7 +11,9 @@ import oracle.oracle as orc
 pytestmark = pytest.mark.gpu
 
 
-@pytest.mark.parametrize("N,K", [(37, 2048), (11264, 2048), (2048, 5632), (5, 16), (300, 32768)])
+@pytest.mark.parametrize("N,K", [(37, 2048), (11264, 2048), (2048, 5632), (5, 16), (300, 32768),
+                                 # K slices that end inside a batch, 2 / 4 / 8 loads per row, 1 / 3 rows left
+                                 (1, 272), (515, 1040), (1001, 3008), (4097, 2064), (9000, 2304)])
 def test_gemv_i8_dev(gpu, N, K):
     import torch
     rng = np.random.default_rng(N + K)
