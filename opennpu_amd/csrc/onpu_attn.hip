@@ -4,7 +4,8 @@
 // optional per-head sink logit that takes probability mass but has no value), out_h = sum_j p_j
 // V[g][j]. fp32 arithmetic; the KV cache is fp32 or bf16 (widened exactly).
 //
-// Split over the sequence; HBM-bound at long context (K and V are read once). k_attn_part:
+// Split over the sequence; HBM-bound at long context (K and V are read once). k_attn_mfma serves a bf16
+// cache, k_attn_part an fp32 one:
 // workgroup (c, g, z) takes rows [c C, c C + C) of kv head g for HG of the query heads that share
 // it (group z), so each K and V row is read once for HG heads. A row is read by LPR = D / 8
 // consecutive lanes, 16 bytes each (one wave instruction covers 64 / LPR consecutive rows), with
@@ -14,6 +15,9 @@
 // and head), sums the row slots of a wave by shuffles and the waves in LDS, and writes the chunk's
 // (max, sum, o[HG][D]). k_attn_combine: per query head, the chunks' partials rescaled to the
 // global max (and the sink) and divided by the total mass.
+#include <algorithm>
+#include <type_traits>
+
 #include "onpu_launch.h"
 
 namespace {
@@ -229,52 +233,369 @@ __global__ __launch_bounds__(AT) void k_attn_part(AttnArgs a) {
     }
 }
 
-// grid Hq, 256 threads: out[h][d] = sum_c e^(m_c - M) o_c[d] / (sum_c e^(m_c - M) l_c + e^(sink - M)).
-// Thread (group gi, d pair dp) sums chunks gi, gi + G, ... (G = 256 / (D / 2) groups), then LDS.
-template <int HG>
-__global__ __launch_bounds__(256) void k_attn_combine(AttnArgs a) {
-    __shared__ float sred[256 * 2];
-    __shared__ float sm[4];
-    __shared__ float fw[ATT_MAX_CH];                 // e^(m_c - M) per chunk
-    const int h = blockIdx.x, g = h / a.rep, hr = h - g * a.rep, z = hr / HG, hh = hr - z * HG, t = threadIdx.x;
-    const int64_t st = HG * (2 + a.D);
-    const float * wp = a.ws + ((int64_t) g * a.ngrp + z) * a.nch * st;
-    float M = a.sinks ? a.sinks[h] : -__builtin_inff();
-    for (int c = t; c < a.nch; c += 256) M = fmaxf(M, wp[c * st + hh]);
-    M = wave_max(M);
-    if ((t & 63) == 0) sm[t >> 6] = M;
-    __syncthreads();
-    M = fmaxf(fmaxf(sm[0], sm[1]), fmaxf(sm[2], sm[3]));
-    float den = 0.f;
-    for (int c = t; c < a.nch; c += 256) {
-        const float mc = wp[c * st + hh];
-        const float f = mc == -__builtin_inff() ? 0.f : expf(mc - M);
-        fw[c] = f;
-        den += f * wp[c * st + HG + hh];
+// ---- bf16 KV: scores on the matrix cores, no workgroup barrier before the end
+// A wave takes 16 KT rows at a time. Bound by VALU work and latency at short context, by HBM at long.
+// (The kernel above, which bf16 took too, spent its time in four barriers, P in LDS per workgroup and a
+// DPP sum per row and head. Both launches, us per call, Hq / Hkv / D at S rows: 32 / 8 / 128 at 8192
+// 17.8 -> 12.9, at 65536 53.6 -> 52.0 (5.2 TB/s); 32 / 4 / 128 at 16384 36.8 -> 14.8; 64 / 8 / 64 at 65536
+// 61.7 -> 30.9; 16 / 2 / 256 at 16384 44.6 -> 22.2; 40 / 8 / 128 at 65536 93.6 -> 53.1. Error against 64 bits at
+// those layouts 1.6-2.2e-7 -> 1.6-1.85e-7.) A row of an
+// MFMA's A operand is one of three bf16 parts of one of 4 heads' q (row 4 h + part): q cut at its bits,
+// 8 + 8 + 8, so the parts sum to q exactly and the products with bf16 K are exact; the steps' sums
+// add as a tree, and the three fp32 sums of a (head, row) end in one lane (16 h + row of the 16), which adds them: no cross-lane sum and
+// one exp per score. p goes through the wave's own LDS to the V layout (8 values of d per lane, LPR
+// lanes per row) and o accumulates in fp32 by v_mfma_f32_4x4x1 (on the VALU for one or two heads), with
+// a running maximum per wave. K of the
+// next pass is loaded after this one's scores, V after this one's products, into the same registers.
+// At the end the row slots of a wave are summed by half-swaps that leave each lane fewer heads, the
+// waves meet in LDS, and a chunk's (max, sum, o) goes to the workspace (or, with one chunk, to out).
+typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
+typedef float f32x4 __attribute__((ext_vector_type(4)));
+constexpr int MT = 256, MW = MT / 64;
+
+// a workgroup barrier that orders LDS accesses only: global loads stay in flight across it
+__device__ __forceinline__ void lds_barrier() {
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup", "local");
+    __builtin_amdgcn_s_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
+}
+
+template <bool MAX> __device__ __forceinline__ float row16(float x) {        // over a row of 16 lanes
+    if (MAX) {
+        x = fmaxf(x, dpp_f<0xB1>(x));
+        x = fmaxf(x, dpp_f<0x4E>(x));
+        x = fmaxf(x, dpp_f<0x141>(x));
+        return fmaxf(x, dpp_f<0x140>(x));
     }
-    den = wave_sum(den);
-    __syncthreads();
-    if ((t & 63) == 0) sm[t >> 6] = den;
-    __syncthreads();
-    den = sm[0] + sm[1] + sm[2] + sm[3] + (a.sinks ? expf(a.sinks[h] - M) : 0.f);
-    const int np = a.D / 2, G = 256 / np, dp = t % np, gi = t / np;
-    float n0 = 0.f, n1 = 0.f;
-    if (gi < G) {
-#pragma unroll 4
-        for (int c = gi; c < a.nch; c += G) {
-            const float2 o = *(const float2 *) (wp + c * st + 2 * HG + hh * a.D + 2 * dp);
-            n0 += fw[c] * o.x;
-            n1 += fw[c] * o.y;
+    return group_sum<16>(x);
+}
+
+// lanes 32 (16) apart: a's sum in the lower, b's in the upper half (of each 32)
+template <int HALF> __device__ __forceinline__ float swap_sum(float a, float b) {
+    typedef unsigned u2 __attribute__((ext_vector_type(2)));
+    const u2 r = HALF == 32 ? __builtin_amdgcn_permlane32_swap(__float_as_uint(a), __float_as_uint(b), false, false)
+                            : __builtin_amdgcn_permlane16_swap(__float_as_uint(a), __float_as_uint(b), false, false);
+    return __uint_as_float(r.x) + __uint_as_float(r.y);
+}
+
+// LDS: P [MW][16 KT][HG], ml [MW][HG][2], red [MW][HG][D] (first the A fragments, 1 KiB each)
+template <int NS, int HG, int KT>
+__global__ __launch_bounds__(MT, 2) void k_attn_mfma(AttnArgs a) {
+    constexpr int LPR = 4 * NS, RPW = 64 / LPR, NSET = (HG + 3) / 4;
+    extern __shared__ __align__(16) float lds[];
+    const int D = a.D, c = blockIdx.x, g = blockIdx.y, z = blockIdx.z;
+    const int lane = threadIdx.x & 63, w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int key = lane & 15, quad = lane >> 4, li = lane % LPR, slot = lane / LPR;
+    float * P = lds + w * 16 * KT * HG, * ml = lds + MW * 16 * KT * HG, * red = ml + 2 * MW * HG;
+    const int64_t j0 = (int64_t) c * a.C;
+    const int rows = (int) (a.S - j0 < a.C ? a.S - j0 : a.C);
+    const uint16_t * Kg = (const uint16_t *) a.K + (int64_t) g * a.hs + j0 * a.rs;
+    const uint16_t * Vg = (const uint16_t *) a.V + (int64_t) g * a.hs + j0 * a.rs + (8 * li < D ? 8 * li : 0);
+    const int hq0 = z * HG, hqn = a.rep - hq0 < HG ? a.rep - hq0 : HG;      // q heads of this group
+    uint4 kr[KT][NS], vr[KT][NS];
+    float mk[KT];
+    // mask values through a buffer that is empty without a mask (no branch: a load under one is
+    // waited for, with everything before it, where the paths meet); K and V rows past the chunk
+    // re-read its last row
+    const __amdgpu_buffer_rsrc_t mr =
+        __builtin_amdgcn_make_buffer_rsrc((void *) (a.mask ? a.mask + j0 : a.q), (short) 0, a.mask ? rows * 4 : 0, 0x00020000);
+    auto load_k = [&](int r0) {
+#pragma unroll
+        for (int t = 0; t < KT; t++)
+            mk[t] = __uint_as_float(__builtin_amdgcn_raw_buffer_load_b32(mr, (uint32_t) (4 * (r0 + 16 * t + key)), 0, 0));
+#pragma unroll
+        for (int t = 0; t < KT; t++) {
+            const int row = r0 + 16 * t + key;
+            const uint16_t * p = Kg + (int64_t) (row < rows ? row : rows - 1) * a.rs;
+#pragma unroll
+            for (int s = 0; s < NS; s++) {                                   // past D: column 0, zeroed below
+                const int d = 32 * s + 8 * quad;
+                kr[t][s] = *(const uint4 *) (p + (d < D ? d : 0));
+            }
+        }
+    };
+    auto load_v = [&](int r0) {
+#pragma unroll
+        for (int t = 0; t < KT; t++)
+#pragma unroll
+            for (int s = 0; s < NS; s++) {
+                const int row = r0 + 16 * t + RPW * s + slot;
+                vr[t][s] = *(const uint4 *) (Vg + (int64_t) (row < rows ? row : rows - 1) * a.rs);
+            }
+    };
+    // A fragments of the scores: lane (row = lane & 15: head row / 4, part row % 4; k = 8 quad + e).
+    // Wave w cuts fragments w, w + 4, ... for all; q is loaded before K and V, so that cutting it
+    // overlaps their latency (the barrier waits for LDS only).
+    constexpr int NF = (NSET * NS + MW - 1) / MW;
+    const int part = key & 3;
+    float4 q4[NF][2];
+    bool qok[NF];
+#pragma unroll
+    for (int i = 0; i < NF; i++) {
+        const int f = w + MW * i, h = 4 * (f / NS) + (key >> 2), d = 32 * (f % NS) + 8 * quad;
+        qok[i] = h < hqn && d < D && part < 3;
+        const float4 * qp = (const float4 *) (a.q + (int64_t) (g * a.rep + hq0) * D + (qok[i] ? h * D + d : 0));
+        q4[i][0] = qp[0];
+        q4[i][1] = qp[1];
+    }
+    __builtin_amdgcn_sched_barrier(0);                           // q's loads stay ahead
+    int r0 = w * 16 * KT;
+    load_k(r0);
+    load_v(r0);
+    const uint32_t cut0 = part >= 1 ? 0xffff0000u : 0u, cut1 = part == 2 ? 0xffff0000u : 0u;
+#pragma unroll
+    for (int i = 0; i < NF; i++) {
+        const float x[8] = {q4[i][0].x, q4[i][0].y, q4[i][0].z, q4[i][0].w, q4[i][1].x, q4[i][1].y, q4[i][1].z, q4[i][1].w};
+        uint32_t u[8];
+#pragma unroll
+        for (int e = 0; e < 8; e++) {                            // x, x - its top part, less that one's
+            const float y = x[e] - __uint_as_float(__float_as_uint(x[e]) & cut0);
+            u[e] = qok[i] ? __float_as_uint(y - __uint_as_float(__float_as_uint(y) & cut1)) : 0u;
+        }
+        if (w + MW * i < NSET * NS)
+            *((uint4 *) red + (w + MW * i) * 64 + lane) =
+                make_uint4(__builtin_amdgcn_perm(u[1], u[0], 0x07060302u), __builtin_amdgcn_perm(u[3], u[2], 0x07060302u),
+                           __builtin_amdgcn_perm(u[5], u[4], 0x07060302u), __builtin_amdgcn_perm(u[7], u[6], 0x07060302u));
+    }
+    lds_barrier();
+    bf16x8 qa[NSET][NS];
+#pragma unroll
+    for (int f = 0; f < NSET * NS; f++) qa[f / NS][f % NS] = __builtin_bit_cast(bf16x8, *((const uint4 *) red + f * 64 + lane));
+    f32x4 av[NSET][8] = {};                                      // o: element h % 4 of av[h / 4][e]
+    float m[NSET], l[NSET];
+#pragma unroll
+    for (int h4 = 0; h4 < NSET; h4++) { m[h4] = -__builtin_inff(); l[h4] = 0.f; }
+
+    auto pass = [&](auto more) {
+        const int rn = r0 + MW * 16 * KT;
+        float sc[KT][NSET];
+#pragma unroll
+        for (int t = 0; t < KT; t++) {
+            f32x4 d[NSET][NS];                                               // a sum per step, added as a tree
+#pragma unroll
+            for (int s = 0; s < NS; s++) {
+                uint4 kv = kr[t][s];
+                if (D < 32 * NS && 32 * s + 8 * quad >= D) kv = make_uint4(0, 0, 0, 0);
+#pragma unroll
+                for (int h4 = 0; h4 < NSET; h4++)
+                    d[h4][s] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(qa[h4][s], __builtin_bit_cast(bf16x8, kv), (f32x4){0, 0, 0, 0}, 0, 0, 0);
+            }
+#pragma unroll
+            for (int h4 = 0; h4 < NSET; h4++)
+#pragma unroll
+                for (int o = 1; o < NS; o *= 2)
+#pragma unroll
+                    for (int s = 0; s < NS; s += 2 * o) d[h4][s] += d[h4][s + o];
+            const int row = r0 + 16 * t + key;
+#pragma unroll
+            for (int h4 = 0; h4 < NSET; h4++) {
+                // (the lower parts' sums are NaN where an infinite K meets their zeros)
+                const f32x4 y = d[h4][0];
+                const float x = y[0] + (__builtin_isfinite(y[0]) ? y[1] + y[2] : 0.f);
+                sc[t][h4] = row < rows ? x * a.scale + mk[t] : -__builtin_inff();
+            }
+        }
+        if (more) load_k(rn);
+        float al[NSET];
+        bool up = false;
+#pragma unroll
+        for (int h4 = 0; h4 < NSET; h4++) {
+            float mx = sc[0][h4];
+#pragma unroll
+            for (int t = 1; t < KT; t++) mx = fmaxf(mx, sc[t][h4]);
+            mx = fmaxf(m[h4], row16<true>(mx));
+            al[h4] = m[h4] == mx ? 1.f : expf(m[h4] - mx);                   // 0 from a first finite maximum
+            up = up || m[h4] != mx;
+            m[h4] = mx;
+            l[h4] *= al[h4];
+#pragma unroll
+            for (int t = 0; t < KT; t++) {
+                const float p = mx == -__builtin_inff() ? 0.f : expf(sc[t][h4] - mx);
+                l[h4] += p;
+                if (4 * h4 + quad < HG) P[(16 * t + key) * HG + 4 * h4 + quad] = p;
+            }
+        }
+        // o of this pass alone, added to the scaled o of those before it: shorter sums, less rounding (not
+        // at 8 heads of D > 128, which have no registers left for both)
+        constexpr bool OWN = NS * HG < 64;
+        float f[HG];
+        const bool rescale = r0 >= MW * 16 * KT && __any(up);                // (the first pass finds o = 0)
+        if (rescale) {
+#pragma unroll
+            for (int h = 0; h < HG; h++) {
+                f[h] = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(al[h / 4]), 16 * (h % 4)));
+#pragma unroll
+                for (int e = 0; e < 8; e++)
+                    if (!OWN) av[h / 4][e][h % 4] *= f[h];
+            }
+        }
+        f32x4 pv[NSET][8];
+#pragma unroll
+        for (int h4 = 0; h4 < NSET; h4++)
+#pragma unroll
+            for (int e = 0; e < 8; e++) pv[h4][e] = OWN ? (f32x4){0, 0, 0, 0} : av[h4][e];
+        if (r0 + 16 * KT > rows) {                                           // rows past the chunk: p = 0, V = 0
+#pragma unroll
+            for (int t = 0; t < KT; t++)
+#pragma unroll
+                for (int s = 0; s < NS; s++)
+                    if (r0 + 16 * t + RPW * s + slot >= rows) vr[t][s] = make_uint4(0, 0, 0, 0);
+        }
+        __builtin_amdgcn_wave_barrier();                                     // the wave's LDS is in order
+#pragma unroll
+        for (int t = 0; t < KT; t++)
+#pragma unroll
+            for (int s = 0; s < NS; s++) {
+                // lane (16 slot + 4 b + c): p of head c (and 4 + c) and V of its own 8 columns; block b of
+                // v_mfma_f32_4x4x1 multiplies the 4 heads by its lanes' columns, fp32, into the lane
+                const float * pp = P + (16 * t + RPW * s + slot) * HG + (HG >= 4 ? lane & 3 : 0);
+                const uint32_t u[4] = {vr[t][s].x, vr[t][s].y, vr[t][s].z, vr[t][s].w};
+#pragma unroll
+                for (int e = 0; e < 8; e++) {
+                    const float v = __uint_as_float(e & 1 ? u[e / 2] & 0xffff0000u : u[e / 2] << 16);
+#pragma unroll
+                    for (int h = 0; h < HG; h += HG >= 4 ? 4 : 1) {
+                        if (HG >= 4) pv[h / 4][e] = __builtin_amdgcn_mfma_f32_4x4x1f32(pp[h], v, pv[h / 4][e], 0, 0, 0);
+                        else pv[0][e][h] += pp[h] * v;
+                    }
+                }
+            }
+#pragma unroll
+        for (int h = 0; h < HG; h++)
+#pragma unroll
+            for (int e = 0; e < 8; e++) {
+                const float o = av[h / 4][e][h % 4], n = pv[h / 4][e][h % 4];
+                av[h / 4][e][h % 4] = !OWN ? n : (rescale ? __builtin_fmaf(o, f[h], n) : o + n);
+            }
+        __builtin_amdgcn_wave_barrier();
+        if (more) load_v(rn);
+        r0 = rn;
+    };
+    while (r0 + MW * 16 * KT < rows) pass(std::true_type{});
+    if (r0 < rows) pass(std::false_type{});
+#pragma unroll
+    for (int h4 = 0; h4 < NSET; h4++) {
+        l[h4] = row16<false>(l[h4]);
+        if (key == 0 && 4 * h4 + quad < HG) {
+            ml[(w * HG + 4 * h4 + quad) * 2] = m[h4];
+            ml[(w * HG + 4 * h4 + quad) * 2 + 1] = l[h4];
         }
     }
-    sred[2 * t] = n0;
-    sred[2 * t + 1] = n1;
+    float acc[HG][8];
+#pragma unroll
+    for (int h = 0; h < HG; h++)
+#pragma unroll
+        for (int e = 0; e < 8; e++) acc[h][e] = av[h / 4][e][h % 4];
+    // sum the row slots; each halving leaves a lane the heads of its half while there are two or more
+    int hb = 0;                                                              // first head of this lane
+    constexpr int H1 = RPW >= 2 && HG >= 2 ? HG / 2 : HG, H2 = RPW >= 4 && H1 >= 2 ? H1 / 2 : H1;
+    if (RPW >= 2) {
+#pragma unroll
+        for (int h = 0; h < H1; h++)
+#pragma unroll
+            for (int e = 0; e < 8; e++) acc[h][e] = swap_sum<32>(acc[h][e], acc[HG >= 2 ? h + H1 : h][e]);
+        if (HG >= 2) hb += (lane >> 5) * H1;
+    }
+    if (RPW >= 4) {
+#pragma unroll
+        for (int h = 0; h < H2; h++)
+#pragma unroll
+            for (int e = 0; e < 8; e++) acc[h][e] = swap_sum<16>(acc[h][e], acc[H1 >= 2 ? h + H2 : h][e]);
+        if (H1 >= 2) hb += ((lane >> 4) & 1) * H2;
+    }
+    if (RPW >= 8) {
+#pragma unroll
+        for (int h = 0; h < H2; h++)
+#pragma unroll
+            for (int e = 0; e < 8; e++) acc[h][e] += dpp_f<0x128>(acc[h][e]);   // row_ror:8
+    }
+    lds_barrier();                                               // every wave has its fragments: red is free
+    if (8 * li < D) {
+#pragma unroll
+        for (int h = 0; h < H2; h++) {
+            float4 * o = (float4 *) (red + (w * HG + hb + h) * D + 8 * li);
+            o[0] = make_float4(acc[h][0], acc[h][1], acc[h][2], acc[h][3]);
+            o[1] = make_float4(acc[h][4], acc[h][5], acc[h][6], acc[h][7]);
+        }
+    }
+    lds_barrier();
+    float * wp = a.ws + (((int64_t) g * a.ngrp + z) * a.nch + c) * (HG * (2 + D));
+    constexpr int DP = 32 * NS;                                  // D rounded up: a power of two
+    const int d = threadIdx.x % DP;
+    for (int h = threadIdx.x / DP; h < HG && d < D; h += MT / DP) {
+        float M = ml[2 * h], sum = 0.f, L = 0.f;
+#pragma unroll
+        for (int k = 1; k < MW; k++) M = fmaxf(M, ml[(k * HG + h) * 2]);
+        const float sink = a.sinks && a.nch == 1 && h < hqn ? a.sinks[g * a.rep + hq0 + h] : -__builtin_inff();
+        M = fmaxf(M, sink);
+#pragma unroll
+        for (int k = 0; k < MW; k++) {
+            const float mk = ml[(k * HG + h) * 2], f = mk == -__builtin_inff() ? 0.f : expf(mk - M);
+            sum += f * red[(k * HG + h) * D + d];
+            L += f * ml[(k * HG + h) * 2 + 1];
+        }
+        if (a.nch == 1) {
+            if (a.sinks) L += expf(sink - M);
+            if (h < hqn) a.out[(int64_t) (g * a.rep + hq0 + h) * D + d] = sum / L;
+            continue;
+        }
+        wp[2 * HG + h * D + d] = sum;
+        if (d == 0) {
+            wp[h] = M;
+            wp[HG + h] = L;
+        }
+    }
+}
+
+// grid (Hq, ceil(D / 64)), 8 waves: out[h][d] = sum_c e^(m_c - M) o_c[d] / (sum_c e^(m_c - M) l_c +
+// e^(sink - M)). A lane per column; every wave finds M and the denominator by itself, a chunk per
+// lane, and sums chunks w, w + 8, ..., 8 o loads at a time; the first 8 go out before M is known, so
+// that one memory latency covers up to 64 chunks. The waves meet in LDS once. Latency-bound (32 heads,
+// 64 chunks: 4.4 us with a workgroup per head in four dependent passes, 2.7-3.8 now).
+constexpr int CW = 8, CB = 8;
+template <int HG>
+__global__ __launch_bounds__(64 * CW) void k_attn_combine(AttnArgs a) {
+    __shared__ float sred[CW][64];
+    const int h = blockIdx.x, g = h / a.rep, hr = h - g * a.rep, z = hr / HG, hh = hr - z * HG;
+    const int lane = threadIdx.x & 63, w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), d = 64 * blockIdx.y + lane;
+    const int64_t st = HG * (2 + a.D);
+    const float * wp = a.ws + ((int64_t) g * a.ngrp + z) * a.nch * st;
+    const float * wo = wp + 2 * HG + hh * a.D + (d < a.D ? d : 0);
+    float ov[CB];
+    auto load_o = [&](int b) {                                   // (past the chunks: the last, unused)
+#pragma unroll
+        for (int k = 0; k < CB; k++) {
+            const int c = b + w + CW * k < a.nch ? b + w + CW * k : a.nch - 1;
+            ov[k] = wo[c * st];
+        }
+    };
+    load_o(0);
+    const int c0 = lane < a.nch ? lane : a.nch - 1;
+    const float m0 = wp[c0 * st + hh], l0 = wp[c0 * st + HG + hh], sink = a.sinks ? a.sinks[h] : -__builtin_inff();
+    float M = fmaxf(m0, sink);
+    for (int c = lane + 64; c < a.nch; c += 64) M = fmaxf(M, wp[c * st + hh]);
+    M = wave_max(M);
+    float den = 0.f, acc = 0.f;
+    for (int b = 0; b < a.nch; b += 64) {
+        const int c = b + lane;
+        const float mc = c >= a.nch ? -__builtin_inff() : (b == 0 ? m0 : wp[c * st + hh]);
+        // (a chunk without a finite score has sum 0 and weight 0)
+        const float f = mc == -__builtin_inff() ? 0.f : expf(mc - M);
+        if (c < a.nch) den += f * (b == 0 ? l0 : wp[c * st + HG + hh]);
+#pragma unroll
+        for (int k = 0; k < CB; k++)
+            if (b + w + CW * k < a.nch)
+                acc += __int_as_float(__builtin_amdgcn_readlane(__float_as_int(f), w + CW * k)) * ov[k];
+        if (b + 64 < a.nch) load_o(b + 64);
+    }
+    sred[w][lane] = acc;
+    den = wave_sum(den) + (a.sinks ? expf(sink - M) : 0.f);
     __syncthreads();
-    if (t < np) {
-        float s0 = 0.f, s1 = 0.f;
-        for (int i = 0; i < G; i++) { s0 += sred[2 * (i * np + t)]; s1 += sred[2 * (i * np + t) + 1]; }
-        a.out[(int64_t) h * a.D + 2 * t] = s0 / den;
-        a.out[(int64_t) h * a.D + 2 * t + 1] = s1 / den;
+    if (w == 0 && d < a.D) {
+        float sum = 0.f;
+#pragma unroll
+        for (int i = 0; i < CW; i++) sum += sred[i][lane];
+        a.out[(int64_t) h * a.D + d] = sum / den;
     }
 }
 
@@ -308,32 +629,40 @@ size_t attn_lds(const AttnPlan & p, int D) {
     return sizeof(float) * ((size_t) p.HG * p.C + (size_t) AW * p.HG * D + 2 * AW * p.HG + (size_t) p.HG * D);
 }
 
-template <typename KV, int LPR, int HG>
+template <bool BF, int NS, int HG>
 hipError_t run_attn(const AttnArgs & a, const AttnPlan & p, hipStream_t s) {
-    k_attn_part<KV, LPR, HG><<<dim3((unsigned) a.nch, (unsigned) a.Hkv, (unsigned) a.ngrp), AT, attn_lds(p, a.D), s>>>(a);
+    const dim3 grid((unsigned) a.nch, (unsigned) a.Hkv, (unsigned) a.ngrp);
+    if (BF) {
+        constexpr int KT = NS >= 8 || HG >= 8 ? 1 : 2;
+        const size_t lds = sizeof(float) * ((size_t) MW * 16 * KT * HG + 2 * MW * HG) +
+                           std::max<size_t>(sizeof(float) * MW * HG * a.D, 1024 * (size_t) NS * ((HG + 3) / 4));
+        k_attn_mfma<NS, HG, KT><<<grid, MT, lds, s>>>(a);
+    } else {
+        k_attn_part<float, 4 * NS, HG><<<grid, AT, attn_lds(p, a.D), s>>>(a);
+    }
     hipError_t e = hipGetLastError();
-    if (e != hipSuccess) return e;
-    k_attn_combine<HG><<<dim3((unsigned) a.Hq), 256, 0, s>>>(a);
+    if (e != hipSuccess || (BF && a.nch == 1)) return e;
+    k_attn_combine<HG><<<dim3((unsigned) a.Hq, (unsigned) (a.D + 63) / 64), 64 * CW, 0, s>>>(a);
     return hipGetLastError();
 }
 
-template <typename KV, int LPR>
+template <bool BF, int NS>
 hipError_t run_attn_hg(const AttnArgs & a, const AttnPlan & p, hipStream_t s) {
     switch (p.HG) {
-    case 1: return run_attn<KV, LPR, 1>(a, p, s);
-    case 2: return run_attn<KV, LPR, 2>(a, p, s);
-    case 4: return run_attn<KV, LPR, 4>(a, p, s);
-    case 8: return run_attn<KV, LPR, 8>(a, p, s);
+    case 1: return run_attn<BF, NS, 1>(a, p, s);
+    case 2: return run_attn<BF, NS, 2>(a, p, s);
+    case 4: return run_attn<BF, NS, 4>(a, p, s);
+    case 8: return run_attn<BF, NS, 8>(a, p, s);
     default: return hipErrorInvalidValue;
     }
 }
 
-template <typename KV>
+template <bool BF>
 hipError_t run_attn_lpr(const AttnArgs & a, const AttnPlan & p, hipStream_t s) {
     switch (p.LPR) {
-    case 8: return run_attn_hg<KV, 8>(a, p, s);
-    case 16: return run_attn_hg<KV, 16>(a, p, s);
-    case 32: return run_attn_hg<KV, 32>(a, p, s);
+    case 8: return run_attn_hg<BF, 2>(a, p, s);
+    case 16: return run_attn_hg<BF, 4>(a, p, s);
+    case 32: return run_attn_hg<BF, 8>(a, p, s);
     default: return hipErrorInvalidValue;
     }
 }
@@ -354,13 +683,21 @@ hipError_t launch_attn_step(const float * q, int Hq, int D, const void * K, cons
     const int64_t al = kv_bf16 ? 8 : 4;             // 16-byte row starts for the vector loads
     if (rs % al || hs % al || ((uintptr_t) K | (uintptr_t) V | (uintptr_t) q) % 16) return hipErrorInvalidValue;
     if (ws_bytes < attn_ws_bytes(Hq, D, Hkv, S)) return hipErrorInvalidValue;
-    const AttnPlan p = attn_plan(Hq, D, Hkv, S);
+    AttnPlan p = attn_plan(Hq, D, Hkv, S);
+    // Four passes (two at D > 128) in one workgroup cost no more than one pass, the second launch and its
+    // read of the partials: 32 / 8 heads, D = 128, 300 and 500 rows 8.2 and 9.5 us against 6.7 + 3.1, a
+    // call 13.4 -> 10.4 us from Python; D = 256, 300 rows in one workgroup 16.9 us against 13.5.
+    const int64_t one = D > 128 ? 128 : (p.HG >= 8 ? 256 : 512);
+    if (kv_bf16 && S <= one) {
+        p.C = (int) S;
+        p.nch = 1;
+    }
     AttnArgs a;
     a.q = q; a.K = K; a.V = V; a.mask = mask; a.sinks = sinks; a.ws = (float *) ws; a.out = out;
     a.S = S; a.hs = hs; a.rs = rs; a.scale = scale;
     a.Hq = Hq; a.D = D; a.Hkv = Hkv; a.rep = Hq / Hkv; a.ngrp = p.ngrp; a.C = p.C; a.nch = p.nch;
     if (Hkv > 65535 || p.ngrp > 65535 || p.nch > ATT_MAX_CH) return hipErrorInvalidValue;
-    return kv_bf16 ? run_attn_lpr<uint16_t>(a, p, s) : run_attn_lpr<float>(a, p, s);
+    return kv_bf16 ? run_attn_lpr<true>(a, p, s) : run_attn_lpr<false>(a, p, s);
 }
 
 // ------------------------------------------------------------------ Gated DeltaNet decode step

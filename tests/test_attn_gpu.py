@@ -80,6 +80,34 @@ def test_attn_step_dev(gpu, kv, Hq, Hkv, D, S, Smax, masked, sinks):
     assert torch.equal(o2, out)
 
 
+@pytest.mark.parametrize("Hq,Hkv,D,S", [
+    (4, 4, 8, 1), (8, 4, 40, 15), (16, 4, 64, 129), (8, 1, 128, 257),          # 1, 2, 4, 8 heads per group
+    (32, 8, 128, 512), (32, 8, 128, 513), (10, 2, 136, 128), (10, 2, 248, 129), # one chunk and its end
+    (3, 3, 256, 700), (6, 3, 128, 2900),
+])
+def test_attn_step_dev_tails(gpu, Hq, Hkv, D, S):
+    """a bf16 cache at the ends of the 16-row steps, of a wave's and of a workgroup's pass and of the
+    one-launch range, with D below its step of 32, masked rows, and a row whose K holds -inf (score
+    -inf for every head: no weight)"""
+    import torch
+    from opennpu_amd.device import attn_step
+    rng = np.random.default_rng(S * 7 + D)
+    q, K, V, mask, sk = _case(rng, Hq, Hkv, D, S, S + 3, "bf16", True, True)
+    q[:, 0] = 0.5
+    Kf = orc.bf2f(K).reshape(Hkv, S + 3, D)
+    mask[S // 2] = 0.25
+    if S > 2:
+        Kf[:, S // 3, 0] = -np.inf
+    K = orc.f2bf_np(Kf).reshape(Hkv, S + 3, D)
+    with np.errstate(invalid="ignore"):
+        ref = orc.attn_step(q, np.ascontiguousarray(K[:, :S]), np.ascontiguousarray(V.reshape(Hkv, S + 3, D)[:, :S]), mask, sk)
+    assert np.isfinite(ref).all()
+    to = lambda a: torch.from_numpy(np.ascontiguousarray(a).view(np.int16)).view(torch.bfloat16).cuda().reshape(Hkv, S + 3, D)[:, :S]
+    out = attn_step(torch.from_numpy(q).cuda(), to(K), to(V), torch.from_numpy(mask).cuda(), torch.from_numpy(sk).cuda())
+    err = np.abs(out.cpu().numpy() - ref).max() / np.abs(ref).max()
+    assert err <= TOL, err
+
+
 def test_attn_step_dev_argument_errors(gpu):
     """rejected on the host, nothing launched: Hq not a multiple of Hkv, D not a multiple of 8,
     more than 16 query heads per kv head, a short workspace"""
