@@ -882,6 +882,26 @@ hipError_t moe_decode_two(Ffn * f, const uint16_t * x, int64_t T, int k, const i
 }
 
 // routed-expert FFN on device data (act 0, no biases): x bf16 [T][H], ids/w [T][k] -> y [T][Nd]
+// k_moe_few (items of 16 rows, workgroups of half the columns, no LDS) against k_moe_gemm for n routed
+// rows: up to 1.5 rows per expert, where nearly every item is one A block anyway, and further where the
+// 8-wave workgroups of gate+up leave CUs idle (us per layer, k_moe_gemm -> k_moe_few, 3 banks in turn):
+//   128 experts, H 2048, I 768, k 8 (768 workgroups): 6 / 24 tokens 44.2 / 75.0 -> 40.4 / 69.2, q4nx
+//     49.1 / 83.6 -> 44.6 / 79.3; 32 tokens (2 rows) 76.1 -> 75.7, q4nx 85.4 -> 87.0; 64 tokens 78.4 -> 79.6
+//   one per CU or fewer, to 5 rows: 32 experts, I 1024, k 4 at 40 tokens 43.1 -> 39.6, at 100 45.6 -> 57.0
+//   one per two CUs, to 12: 8 experts, H 4096, I 2048, k 2 at 10 / 40 tokens 57.9 / 59.0 -> 39.6 / 41.1,
+//     at 64 64.3 -> 66.0
+bool moe_few(int64_t n, int64_t E, int64_t I) {
+    const int64_t cus = device().cus > 0 ? device().cus : 256, wgs = E * ((I / 16 + 7) / 8);
+    return 2 * n <= 3 * E || (wgs <= cus && n <= 5 * E) || (2 * wgs <= cus && n <= 12 * E);
+}
+
+// Non-temporal weight loads for a bank of more than 96 MiB, which no 256 MiB last-level cache keeps from
+// one call to the next beside the rest of a model, while an expert's weights are read about once
+// (us per layer, plain -> non-temporal): 311 MB at 24 / 64 / 128 / 700 tokens 74.6 / 82.3 / 83.8 / 115.6 ->
+// 69.2 / 78.4 / 80.5 / 114.6, q4nx (377 MB) at 128 101.8 -> 91.3; at 1000 tokens (62 rows per expert, many
+// read twice) 157.3 -> 161.0. Banks of 78 and 13 MB, which stay cached: 32.0 -> 34.2, 27.1 -> 28.5.
+bool moe_nt(int64_t n, int64_t E, int64_t bytes) { return bytes > ((int64_t) 96 << 20) && n <= 48 * E; }
+
 hipError_t ffn_core(Ffn * f, const uint16_t * x, int64_t T, const int32_t * ids, int k, const float * w, void * y,
                     int yf32, hipStream_t s) {
     Mat4 * gu = f->gu, * dn = f->dn;
@@ -899,8 +919,10 @@ hipError_t ffn_core(Ffn * f, const uint16_t * x, int64_t T, const int32_t * ids,
         return moe_decode_two(f, x, T, k, ids, w, y, yf32, s);
     }
     // prompts: tokens grouped per expert (one pass over each routed expert's weights per 64 rows)
-    const int rows_per_item = 64;                 // the grouped GEMM's 4 A blocks of 16 rows
-    const int64_t E = gu->E, maxitems = n / rows_per_item + E;
+    const int64_t E = gu->E;
+    const bool few = moe_few(n, E, I), nt = moe_nt(n, E, E * (gu->dstride + dn->dstride));
+    const int rows_per_item = few ? 16 : 64;      // one A block, or the grouped GEMM's 4
+    const int64_t maxitems = n / rows_per_item + E;
     if ((e = f->ws[1].ensure((size_t) (E + 1) * 4)) != hipSuccess) return e;
     if ((e = f->ws[2].ensure((size_t) n * 4)) != hipSuccess) return e;
     if ((e = f->ws[3].ensure((size_t) n * 4)) != hipSuccess) return e;
@@ -917,13 +939,15 @@ hipError_t ffn_core(Ffn * f, const uint16_t * x, int64_t T, const int32_t * ids,
     a.W = gu->dev; a.estride = gu->dstride; a.NT = gu->g.NT; a.KB = gu->g.KB; a.N = gu->N; a.K = gu->K;
     a.x = x; a.ldx = gu->K; a.y = act; a.ldy = I; a.perm = perm; a.items = items; a.nitems = nitems; a.k = k;
     a.xbytes = T * gu->K * 2;
+    a.nt = nt;
     // grouped GEMMs: X tiles in LDS, weights dequantized in registers
     MArgs b{};
     b.W = dn->dev; b.estride = dn->dstride; b.NT = dn->g.NT; b.KB = dn->g.KB; b.N = Nd; b.K = dn->K;
     b.x = act; b.ldx = I; b.y = o; b.ldy = Nd; b.perm = perm; b.items = items; b.nitems = nitems; b.k = k;
     b.xbytes = n * I * 2;
-    if ((e = launch_moe_gemm(gu->fmt, 0, a, maxitems, s)) != hipSuccess) return e;
-    if ((e = launch_moe_gemm(dn->fmt, 1, b, maxitems, s)) != hipSuccess) return e;
+    b.nt = nt;
+    if ((e = launch_moe_gemm(gu->fmt, 0, a, maxitems, few, s)) != hipSuccess) return e;
+    if ((e = launch_moe_gemm(dn->fmt, 1, b, maxitems, few, s)) != hipSuccess) return e;
     return launch_moe_combine(o, inv, w, T, k, Nd, y, yf32, s);
 }
 

@@ -101,14 +101,22 @@ hipError_t FN(relayout_dec)(const uint8_t * src, int64_t sstride, int64_t NT, in
     return hipGetLastError();
 }
 
-hipError_t FN(moe_gemm)(int which, const MArgs & a, dim3 grid, hipStream_t s) {
+template <int WHICH, bool KT>
+static void moe_gemm_wk(bool few, const MArgs & a, dim3 grid, hipStream_t s) {
+    if (few && a.nt) k_moe_few<F, WHICH, KT, 2><<<grid, 64 * MFEW_WV, 0, s>>>(a);
+    else if (few) k_moe_few<F, WHICH, KT, 0><<<grid, 64 * MFEW_WV, 0, s>>>(a);
+    else if (a.nt) k_moe_gemm<F, WHICH, KT, 2><<<grid, 512, 0, s>>>(a);
+    else k_moe_gemm<F, WHICH, KT, 0><<<grid, 512, 0, s>>>(a);
+}
+
+hipError_t FN(moe_gemm)(int which, bool few, const MArgs & a, dim3 grid, hipStream_t s) {
     const bool kt = a.K % 128 != 0;
     if (which == 0) {
-        if (kt) k_moe_gemm<F, 0, true><<<grid, 512, 0, s>>>(a);
-        else k_moe_gemm<F, 0, false><<<grid, 512, 0, s>>>(a);
+        if (kt) moe_gemm_wk<0, true>(few, a, grid, s);
+        else moe_gemm_wk<0, false>(few, a, grid, s);
     } else {
-        if (kt) k_moe_gemm<F, 1, true><<<grid, 512, 0, s>>>(a);
-        else k_moe_gemm<F, 1, false><<<grid, 512, 0, s>>>(a);
+        if (kt) moe_gemm_wk<1, true>(few, a, grid, s);
+        else moe_gemm_wk<1, false>(few, a, grid, s);
     }
     return hipGetLastError();
 }

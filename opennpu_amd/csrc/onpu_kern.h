@@ -1044,28 +1044,30 @@ DEV void gemm_load_x(const __amdgpu_buffer_rsrc_t & xr, const uint32_t (&xo)[MB]
 
 // weight block b of the wave's NTW tiles (buffer loads: one lane offset, the block in the scalar offset)
 // weight tile block b (16 B of codes per lane) and its group parameters for lane row r
-template <int FMT>
-DEV void gemm_load_w1(const __amdgpu_buffer_rsrc_t & wrs, int64_t b, int lane, int r, u32x4 & w, GPar<FMT> & p) {
+// (past: 0, or 0x80000000 to read zeros from past the buffer; AUX: cache policy bits)
+template <int FMT, int AUX = 0>
+DEV void gemm_load_w1(const __amdgpu_buffer_rsrc_t & wrs, int64_t b, int lane, int r, u32x4 & w, GPar<FMT> & p,
+                      uint32_t past = 0u) {
     constexpr int BLK = 1024 + 16 * (128 / (FMT == ONPU_G128S ? 128 : 32)) * 2 * (FMT == ONPU_Q4NX ? 2 : 1);
     const uint32_t sb = (uint32_t) (b * BLK);
-    w = __builtin_bit_cast(u32x4, __builtin_amdgcn_raw_buffer_load_b128(wrs, 16 * lane, sb, 0));
+    w = __builtin_bit_cast(u32x4, __builtin_amdgcn_raw_buffer_load_b128(wrs, (uint32_t) (16 * lane) | past, sb, AUX));
     if (FMT == ONPU_G128S) {
-        p.v[0] = __builtin_amdgcn_raw_buffer_load_b16(wrs, 1024 + 2 * r, sb, 0);
+        p.v[0] = __builtin_amdgcn_raw_buffer_load_b16(wrs, (uint32_t) (1024 + 2 * r) | past, sb, AUX);
     } else if (FMT == ONPU_Q4NX) {
-        const u32x4 v = __builtin_bit_cast(u32x4, __builtin_amdgcn_raw_buffer_load_b128(wrs, 1024 + 16 * r, sb, 0));
+        const u32x4 v = __builtin_bit_cast(u32x4, __builtin_amdgcn_raw_buffer_load_b128(wrs, (uint32_t) (1024 + 16 * r) | past, sb, AUX));
         for (int jj = 0; jj < 4; jj++) p.v[jj % (sizeof(p.v) / 4)] = v[jj];
     } else {
-        const u32x2 v = __builtin_bit_cast(u32x2, __builtin_amdgcn_raw_buffer_load_b64(wrs, 1024 + 8 * r, sb, 0));
+        const u32x2 v = __builtin_bit_cast(u32x2, __builtin_amdgcn_raw_buffer_load_b64(wrs, (uint32_t) (1024 + 8 * r) | past, sb, AUX));
         p.v[0] = v.x;
         p.v[1 % (sizeof(p.v) / 4)] = v.y;
     }
 }
 
-template <int FMT, int NTW>
+template <int FMT, int NTW, int AUX = 0>
 DEV void gemm_load_w(const __amdgpu_buffer_rsrc_t (&wrs)[NTW], int64_t b, int lane, int r, u32x4 (&w)[NTW],
                      GPar<FMT> (&p)[NTW]) {
 #pragma unroll
-    for (int i = 0; i < NTW; i++) gemm_load_w1<FMT>(wrs[i], b, lane, r, w[i], p[i]);
+    for (int i = 0; i < NTW; i++) gemm_load_w1<FMT, AUX>(wrs[i], b, lane, r, w[i], p[i]);
 }
 
 // AK: one row tile (M <= 16 MB), no split: the epilogue also leaves the workgroup's argmax key of
@@ -1619,6 +1621,48 @@ __global__ __launch_bounds__(64 * WV, 1) void k_qgemm_sk(GArgs a) {
     }
 }
 
+// an item's accumulators (lane (q, r): rows 4 q + v of A block mb, column r of tiles t[0], t[1]) to y
+template <int WHICH, int MBG>
+DEV void moe_store(const MArgs & a, int32_t first, int32_t rows, const int64_t (&t)[2], bool ok0, bool ok1,
+                   const f32x4 (&acc)[MBG][2]) {
+    const int lane = threadIdx.x & 63, r = lane & 15, q = lane >> 4;
+    // bf16 stores through a buffer resource over the item's rows (rows <= 64: 32-bit offsets): the
+    // lane's row 4 q and column in the vector offset, the row step 16 mb + v in the scalar offset;
+    // a row past the item or a column past N gets an offset past the range, so the store is dropped
+    const uint32_t rowb = (uint32_t) a.ldy * 2;
+    const __amdgpu_buffer_rsrc_t yr = __builtin_amdgcn_make_buffer_rsrc(
+        (void *) ((uint16_t *) a.y + (int64_t) first * a.ldy), (short) 0, (int) ((uint32_t) rows * rowb), 0x00020000);
+    const int rows_l = rows - 4 * q;                               // rows left from the lane's first
+    uint32_t vo[2];
+#pragma unroll
+    for (int i = 0; i < 2; i++) {
+        const bool okc = (i == 0 ? ok0 : ok1) && 16 * t[i] + r < a.N;
+        vo[i] = okc ? (uint32_t) (4 * q) * rowb + (uint32_t) (16 * t[i] + r) * 2 : 0x80000000u;
+    }
+    // lane (q, r) holds rows 4 q + v of A block mb, column r of its tiles
+#pragma unroll
+    for (int mb = 0; mb < MBG; mb++)
+#pragma unroll
+        for (int v = 0; v < 4; v += 2) {
+            const uint32_t so0 = (uint32_t) (16 * mb + v) * rowb, so1 = so0 + rowb;
+            const bool in0 = 16 * mb + v < rows_l, in1 = 16 * mb + v + 1 < rows_l;
+            if (WHICH == 0) {
+                const uint32_t pk = pack_bf16x2(silu_f(acc[mb][0][v]) * acc[mb][1][v],
+                                                silu_f(acc[mb][0][v + 1]) * acc[mb][1][v + 1]);
+                __builtin_amdgcn_raw_buffer_store_b16((unsigned short) pk, yr, in0 ? vo[0] : 0x80000000u, so0, 0);
+                __builtin_amdgcn_raw_buffer_store_b16((unsigned short) (pk >> 16), yr, in1 ? vo[0] : 0x80000000u, so1, 0);
+            } else {
+#pragma unroll
+                for (int i = 0; i < 2; i++) {
+                    const uint32_t pk = pack_bf16x2(acc[mb][i][v], acc[mb][i][v + 1]);
+                    __builtin_amdgcn_raw_buffer_store_b16((unsigned short) pk, yr, in0 ? vo[i] : 0x80000000u, so0, 0);
+                    __builtin_amdgcn_raw_buffer_store_b16((unsigned short) (pk >> 16), yr, in1 ? vo[i] : 0x80000000u,
+                                                          so1, 0);
+                }
+            }
+        }
+}
+
 // ------------------------------------------------------------------ MoE prefill: grouped GEMM
 // Work item = (expert e, first permuted position, rows <= 64) from k_moe_permute, taken with a group
 // cg of output columns by each workgroup (k_moe_gemm below maps workgroups to (item, cg) so that an
@@ -1636,7 +1680,7 @@ __global__ __launch_bounds__(64 * WV, 1) void k_qgemm_sk(GArgs a) {
 //           reference device's output precision per expert: its GEMV flushes each row to bf16,
 //           gemv_any.cc:120-130, and the host sums the weighted rows in fp32, onpu_cpu.cpp:259-274)
 // X rows: WHICH 0 token perm[position] / k of x [T][K]; WHICH 1 position of act [T k][K].
-template <int FMT, int WHICH, int WV, int MBG, bool KT>
+template <int FMT, int WHICH, int WV, int MBG, bool KT, int AUX>
 DEV void moe_gemm_item(const MArgs & a, int64_t cg, int32_t e, int32_t first, int32_t rows, u32x4 * xs0, u32x4 * xs1) {
     // X fragments f = FPW wave + i (i < FPW, f < 4 MBG): (mb, j) = (f / 4, f % 4); FPW divides 4,
     // so that a wave's fragments share one A block and each lane one row
@@ -1685,64 +1729,31 @@ DEV void moe_gemm_item(const MArgs & a, int64_t cg, int32_t e, int32_t first, in
     u32x4 wa[2], wb[2];
     GPar<FMT> pa[2], pb[2];
     load_xt(0, xs0);
-    gemm_load_w<FMT, 2>(wrs, 0, lane, r, wa, pa);
+    gemm_load_w<FMT, 2, AUX>(wrs, 0, lane, r, wa, pa);
     __builtin_amdgcn_s_waitcnt(0x0f70);
     __syncthreads();
     int64_t b = 0;
     for (; b + 2 <= a.KB; b += 2) {
         load_xt(b + 1, xs1);
-        gemm_load_w<FMT, 2>(wrs, b + 1, lane, r, wb, pb);
+        gemm_load_w<FMT, 2, AUX>(wrs, b + 1, lane, r, wb, pb);
         gemm_block<FMT, 2, MBG>(xs0, wa, pa, lane, acc);
         __builtin_amdgcn_s_waitcnt(0x0f70);
         __syncthreads();
         if (b + 2 < a.KB) {
             load_xt(b + 2, xs0);
-            gemm_load_w<FMT, 2>(wrs, b + 2, lane, r, wa, pa);
+            gemm_load_w<FMT, 2, AUX>(wrs, b + 2, lane, r, wa, pa);
         }
         gemm_block<FMT, 2, MBG>(xs1, wb, pb, lane, acc);
         __builtin_amdgcn_s_waitcnt(0x0f70);
         __syncthreads();
     }
     if (b < a.KB) gemm_block<FMT, 2, MBG>(xs0, wa, pa, lane, acc);
-    // bf16 stores through a buffer resource over the item's rows (rows <= 64: 32-bit offsets): the
-    // lane's row 4 q and column in the vector offset, the row step 16 mb + v in the scalar offset;
-    // a row past the item or a column past N gets an offset past the range, so the store is dropped
-    const uint32_t rowb = (uint32_t) a.ldy * 2;
-    const __amdgpu_buffer_rsrc_t yr = __builtin_amdgcn_make_buffer_rsrc(
-        (void *) ((uint16_t *) a.y + (int64_t) first * a.ldy), (short) 0, (int) ((uint32_t) rows * rowb), 0x00020000);
-    const int rows_l = rows - 4 * q;                               // rows left from the lane's first
-    uint32_t vo[2];
-#pragma unroll
-    for (int i = 0; i < 2; i++) {
-        const bool okc = (i == 0 ? ok0 : ok1) && 16 * t[i] + r < a.N;
-        vo[i] = okc ? (uint32_t) (4 * q) * rowb + (uint32_t) (16 * t[i] + r) * 2 : 0x80000000u;
-    }
-    // lane (q, r) holds rows 4 q + v of A block mb, column r of its tiles
-#pragma unroll
-    for (int mb = 0; mb < MBG; mb++)
-#pragma unroll
-        for (int v = 0; v < 4; v += 2) {
-            const uint32_t so0 = (uint32_t) (16 * mb + v) * rowb, so1 = so0 + rowb;
-            const bool in0 = 16 * mb + v < rows_l, in1 = 16 * mb + v + 1 < rows_l;
-            if (WHICH == 0) {
-                const uint32_t pk = pack_bf16x2(silu_f(acc[mb][0][v]) * acc[mb][1][v],
-                                                silu_f(acc[mb][0][v + 1]) * acc[mb][1][v + 1]);
-                __builtin_amdgcn_raw_buffer_store_b16((unsigned short) pk, yr, in0 ? vo[0] : 0x80000000u, so0, 0);
-                __builtin_amdgcn_raw_buffer_store_b16((unsigned short) (pk >> 16), yr, in1 ? vo[0] : 0x80000000u, so1, 0);
-            } else {
-#pragma unroll
-                for (int i = 0; i < 2; i++) {
-                    const uint32_t pk = pack_bf16x2(acc[mb][i][v], acc[mb][i][v + 1]);
-                    __builtin_amdgcn_raw_buffer_store_b16((unsigned short) pk, yr, in0 ? vo[i] : 0x80000000u, so0, 0);
-                    __builtin_amdgcn_raw_buffer_store_b16((unsigned short) (pk >> 16), yr, in1 ? vo[i] : 0x80000000u,
-                                                          so1, 0);
-                }
-            }
-        }
+    moe_store<WHICH, MBG>(a, first, rows, t, ok0, ok1, acc);
 }
 
 // KT: K % 128 != 0 (launched with KT = false otherwise, so that no block pays for the tail check)
-template <int FMT, int WHICH, bool KT>
+// AUX: cache policy of the weight loads (2: non-temporal; MArgs::nt)
+template <int FMT, int WHICH, bool KT, int AUX>
 // grid: (column groups G, item slots, a multiple of 8). Workgroup L = x + G y runs on XCD L % 8; its
 // position j = L / 8 there takes item 8 (j / G) + L % 8 and column group j % G, so the G column
 // groups of an item run together on one XCD and fetch the item's X rows into that XCD's L2 once
@@ -1755,12 +1766,87 @@ __global__ __launch_bounds__(512, 1) void k_moe_gemm(MArgs a) {
     const int64_t cg = j % G;
     if (item >= *a.nitems) return;
     const int32_t e = a.items[3 * item], first = a.items[3 * item + 1], rows = a.items[3 * item + 2];
-    if (rows <= 16) moe_gemm_item<FMT, WHICH, WV, 1, KT>(a, cg, e, first, rows, xs0, xs1);
-    else if (rows <= 32) moe_gemm_item<FMT, WHICH, WV, 2, KT>(a, cg, e, first, rows, xs0, xs1);
-    else if (rows <= 48) moe_gemm_item<FMT, WHICH, WV, 3, KT>(a, cg, e, first, rows, xs0, xs1);
-    else moe_gemm_item<FMT, WHICH, WV, 4, KT>(a, cg, e, first, rows, xs0, xs1);
+    if (rows <= 16) moe_gemm_item<FMT, WHICH, WV, 1, KT, AUX>(a, cg, e, first, rows, xs0, xs1);
+    else if (rows <= 32) moe_gemm_item<FMT, WHICH, WV, 2, KT, AUX>(a, cg, e, first, rows, xs0, xs1);
+    else if (rows <= 48) moe_gemm_item<FMT, WHICH, WV, 3, KT, AUX>(a, cg, e, first, rows, xs0, xs1);
+    else moe_gemm_item<FMT, WHICH, WV, 4, KT, AUX>(a, cg, e, first, rows, xs0, xs1);
 }
 
+
+// The grouped products of items of at most 16 rows (small batches over many experts, or few
+// workgroups in all: the host's moe_few() rule). Nearly all of the time is the weights' dequant (one
+// MFMA per fragment) and their bytes. Four waves x 2 weight tiles, no LDS and no barrier: each wave
+// brings its own X fragments to registers with the weights of the same block, two register sets in
+// turn, and runs free with one to two blocks in flight; five workgroups fit a CU (24 tokens over
+// 128 experts: gate+up 40.9 -> 36, down 26.3 -> 21 us with non-temporal loads). Blocks past
+// the last are loaded from past the buffers, as zeros, and add zero: no branch, so that the compiler's
+// waits stay exact. Same numbers as k_moe_gemm (the products of a row in the same order).
+constexpr int MFEW_WV = 4;
+template <int FMT, int WHICH, bool KT, int AUX>
+__global__ __launch_bounds__(64 * MFEW_WV, 5) void k_moe_few(MArgs a) {
+    constexpr int WV = MFEW_WV, BLK = 1024 + 16 * (128 / (FMT == ONPU_G128S ? 128 : 32)) * 2 * (FMT == ONPU_Q4NX ? 2 : 1);
+    const int64_t G = gridDim.x, L = blockIdx.x + G * blockIdx.y, cg = (L / 8) % G;
+    const int item = (int) (8 * (L / 8 / G) + L % 8);            // as k_moe_gemm: an item's columns on one XCD
+    if (item >= *a.nitems) return;
+    const int32_t e = a.items[3 * item], first = a.items[3 * item + 1], rows = a.items[3 * item + 2];
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), r = lane & 15, q = lane >> 4;
+    const uint8_t * W = a.W + (int64_t) e * a.estride;
+    int64_t t[2];
+    if (WHICH == 0) { t[0] = cg * WV + wave; t[1] = t[0] + a.NT / 2; }
+    else { t[0] = cg * 2 * WV + 2 * wave; t[1] = t[0] + 1; }
+    if (t[0] >= (WHICH == 0 ? a.NT / 2 : a.NT)) return;
+    const bool ok1 = t[1] < a.NT;
+    __amdgpu_buffer_rsrc_t wrs[2];
+    for (int i = 0; i < 2; i++)
+        wrs[i] = __builtin_amdgcn_make_buffer_rsrc((void *) (W + (i == 0 || ok1 ? t[i] : t[0]) * a.KB * BLK), (short) 0,
+                                                   (int) (uint32_t) (a.KB * BLK), 0x00020000);
+    const __amdgpu_buffer_rsrc_t xr =
+        __builtin_amdgcn_make_buffer_rsrc((void *) a.x, (short) 0, (int) (uint32_t) a.xbytes, 0x00020000);
+    uint32_t xrow = 0x80000000u;                                 // rows past the item read zeros
+    if (r < rows) {
+        const int64_t src = WHICH == 0 ? (int64_t) (a.perm[first + r] / a.k) : (int64_t) (first + r);
+        xrow = (uint32_t) (src * a.ldx * 2) + 16u * q;
+    }
+    struct Set { u32x4 w[2], x[4]; GPar<FMT> p[2]; } sa, sb;
+    const int KB = (int) a.KB;
+    auto load = [&](int b, Set & st) {
+        const uint32_t past = b < KB ? 0u : 0x80000000u;
+        const int64_t bi = b < KB ? b : 0;
+#pragma unroll
+        for (int i = 0; i < 2; i++) gemm_load_w1<FMT, AUX>(wrs[i], bi, lane, r, st.w[i], st.p[i], past);
+#pragma unroll
+        for (int j = 0; j < 4; j++) {
+            uint32_t off = xrow | past;
+            if (KT && 128 * b + 32 * j + 8 * q >= a.K) off = 0x80000000u;
+            st.x[j] = __builtin_bit_cast(u32x4, __builtin_amdgcn_raw_buffer_load_b128(xr, off, (uint32_t) (256 * bi + 64 * j), 0));
+        }
+    };
+    f32x4 acc[1][2] = {};
+    auto block = [&](const Set & st) {
+#pragma unroll
+        for (int j = 0; j < 4; j++)
+#pragma unroll
+            for (int i = 0; i < 2; i++) {
+                float sc, cc;
+                par_sc<FMT>(st.p[i], j, sc, cc);
+                acc[0][i] = mfma(st.x[j], dequant8<FMT>(st.w[i][j], sc, cc), acc[0][i]);
+            }
+    };
+    load(0, sa);
+    __builtin_amdgcn_sched_barrier(0);
+    load(1, sb);
+    for (int b = 0; b < KB; b += 2) {
+        block(sa);
+        __builtin_amdgcn_sched_barrier(0);
+        load(b + 2, sa);
+        __builtin_amdgcn_sched_barrier(0);
+        block(sb);
+        __builtin_amdgcn_sched_barrier(0);
+        load(b + 3, sb);
+        __builtin_amdgcn_sched_barrier(0);
+    }
+    moe_store<WHICH, 1>(a, first, rows, t, true, ok1, acc);
+}
 
 // ------------------------------------------------------------------ MoE decode in one launch
 // Opt-in (ONPU_MOE_FUSED=1): measured on MI355X for Qwen3-30B-A3B at T = 1 it takes ~19 us against

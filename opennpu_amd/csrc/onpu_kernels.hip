@@ -536,17 +536,17 @@ hipError_t launch_relayout_dec(int fmt, const uint8_t * src, int64_t sstride, in
     return hipErrorInvalidValue;
 }
 
-hipError_t launch_moe_gemm(int fmt, int which, const MArgs & a, int64_t maxitems, hipStream_t s) {
+hipError_t launch_moe_gemm(int fmt, int which, const MArgs & a, int64_t maxitems, bool few, hipStream_t s) {
     if (a.xbytes <= 0 || a.xbytes >= ((int64_t) 1 << 31) || maxitems <= 0 || maxitems > 65528) return hipErrorInvalidValue;
     if (which == 0 && (a.NT % 2 || a.N != 16 * a.NT)) return hipErrorInvalidValue;   // gate | up halves of whole tiles
-    constexpr int wv = 8;                                   // k_moe_gemm: 8 waves x 2 weight tiles
+    const int wv = few ? 4 : 8;                             // k_moe_few, k_moe_gemm: waves of 2 weight tiles
     const int64_t gx = which == 0 ? (a.NT / 2 + wv - 1) / wv : (a.NT + 2 * wv - 1) / (2 * wv);
     const dim3 grid((unsigned) gx, (unsigned) ((maxitems + 7) / 8 * 8));   // item slots: whole XCD rounds
     switch (fmt) {
-        case 0: return moe_gemm_f0(which, a, grid, s);
-        case 1: return moe_gemm_f1(which, a, grid, s);
-        case 2: return moe_gemm_f2(which, a, grid, s);
-        case 3: return moe_gemm_f3(which, a, grid, s);
+        case 0: return moe_gemm_f0(which, few, a, grid, s);
+        case 1: return moe_gemm_f1(which, few, a, grid, s);
+        case 2: return moe_gemm_f2(which, few, a, grid, s);
+        case 3: return moe_gemm_f3(which, few, a, grid, s);
     }
     return hipErrorInvalidValue;
 }

@@ -84,6 +84,7 @@ struct MArgs {
     const int32_t * nitems;
     int k;
     int64_t xbytes;           // k_moe_gemm: bytes of x (buffer range of the gathered rows, < 2^31)
+    int nt;                   // non-temporal weight loads
 };
 
 // MoE decode in one launch (k_moe_decode): router (optional), gate_up + SiLU * up per routed slot,
@@ -197,8 +198,9 @@ hipError_t launch_route(const float * logits, int64_t T, int E, int k, int renor
 // ... and inv[i] = the position of entry i (perm's inverse)
 hipError_t launch_moe_permute(const int32_t * ids, int64_t n, int E, int rows_per_item, int32_t * off, int32_t * perm,
                               int32_t * inv, int32_t * items, int32_t * nitems, hipStream_t s);
-// grouped GEMM over the work items (k_moe_gemm): grid.x column groups (gate_up: NT / 8, down: NT / 8)
-hipError_t launch_moe_gemm(int fmt, int which, const MArgs & a, int64_t maxitems, hipStream_t s);
+// grouped GEMM over the work items: k_moe_gemm (items of up to 64 rows, grid.x column groups of 8 waves x
+// 2 tiles) or few: k_moe_few (items of up to 16 rows, 4 waves)
+hipError_t launch_moe_gemm(int fmt, int which, const MArgs & a, int64_t maxitems, bool few, hipStream_t s);
 // one-launch MoE decode on `grid` workgroups (one per CU); hipErrorInvalidValue when the shapes are
 // outside what k_moe_decode handles (moe_decode_fits; the caller then uses the multi-launch path)
 hipError_t launch_moe_decode(int fmt, const MDArgs & a, int grid, hipStream_t s);
@@ -295,7 +297,7 @@ enum { EPI_STORE_ = 0, EPI_ACT_ = 1, EPI_SLOTSUM_ = 2, EPI_ARGMAX_ = 3 };
                            size_t lds, hipStream_t s);                                                    \
     hipError_t qgemm_f##id(const GArgs & a, int ntw, int mb, hipStream_t s);                                       \
     hipError_t qgemm_sk_f##id(const GArgs & a, int cfg, int grid, hipStream_t s);                          \
-    hipError_t moe_gemm_f##id(int which, const MArgs & a, dim3 grid, hipStream_t s);                  \
+    hipError_t moe_gemm_f##id(int which, bool few, const MArgs & a, dim3 grid, hipStream_t s);        \
     hipError_t moe_decode_f##id(const MDArgs & a, int gb, int grid, size_t lds, hipStream_t s);       \
     hipError_t moe_dsplit_f##id(const MSArgs & a, int nw, int sv, size_t lds, hipStream_t s);         \
     hipError_t relayout_dec_f##id(const uint8_t * src, int64_t sstride, int64_t NT, int64_t KB, uint8_t * dst, \

@@ -120,6 +120,31 @@ def test_moe_grouped_item_sizes(gpu, fmt):
     check_moe(y, fmt, gu, dn, E, H, I, xb, rid, rw, grouped=True, what=f"moe item sizes fmt {fmt}")
 
 
+@pytest.mark.parametrize("fmt", [orc.FMT_G128S, orc.FMT_Q4S, orc.FMT_Q4NX, orc.FMT_Q4_0])
+@pytest.mark.parametrize("H,I", [(256, 128), (384, 256), (288, 160)])
+def test_moe_few_rows_items(gpu, fmt, H, I):
+    """the kernel of few rows per expert (items of at most 16 rows): 1 to 33 rows per expert, so items
+    of 1, 15 and 16 rows and experts of two and three items, one and three K blocks, column groups
+    past the last tile, and (per 32) K tails"""
+    import torch
+    if fmt == orc.FMT_G128S and H % 128:
+        pytest.skip("g128s takes K in multiples of 128")
+    counts = [1, 2, 4, 5, 8, 15, 16, 17, 32, 33] + [0, 1] * 4
+    E, k, T = len(counts), 1, sum(counts)
+    assert T <= 12 * E
+    rng = np.random.default_rng(9)
+    rid = rng.permutation(np.repeat(np.arange(E, dtype=np.int32), counts)).reshape(T, k)
+    rw = rng.uniform(0.5, 1.0, (T, k)).astype(np.float32)
+    gu, dn = _experts(fmt, E, H, I, 6000)
+    xb = syn.activations(T, H, 6)
+    f = _ffn(fmt, E, H, I, gu, dn)
+    try:
+        y = from_torch(f.ffn(to_torch_bf16(xb).reshape(T, H), torch.from_numpy(rid).cuda(), torch.from_numpy(rw).cuda()))
+    finally:
+        f.free()
+    check_moe(y, fmt, gu, dn, E, H, I, xb, rid, rw, grouped=True, what=f"moe few rows fmt {fmt}")
+
+
 @pytest.mark.parametrize("fmt", [orc.FMT_Q4S, orc.FMT_Q4NX])
 def test_moe_grouped_k_tail(gpu, fmt):
     """grouped products whose K is not a multiple of 128 (H = 288 for gate+up, I = 160 for down):
