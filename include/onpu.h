@@ -163,7 +163,7 @@ int onpu_dense_mv_dev(void * h, const void * x, int64_t M, void * y, int y_f32, 
 /* 1 if a split-K GEMM gave up waiting for its partner workgroup since the last call (the flag is then
  * cleared and that launch's Y is invalid), 0 if not, -1 on error; synchronises the device */
 int onpu_gemm_status(void);
-/* frees the device staging of the host-pointer calls (it grows to the largest call; one set for the
+/* frees the device staging and the pinned memory of the host-pointer calls (it grows to the largest call; one set for the
  * library, shared by every handle) */
 void onpu_release_scratch(void);
 /* logits fp32 [M][N] and argmax [M] (first maximum) */

@@ -598,6 +598,18 @@ hipError_t launch_moe_combine(const uint16_t * o, const int32_t * inv, const flo
     return hipSuccess;
 }
 
+// the end of a host-pointer call: everything before it on the stream has completed, and is made visible
+// to the host before the word
+__global__ void k_host_word(uint32_t * word, uint32_t tag) {
+    __hip_atomic_store(word, tag, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
+}
+
+hipError_t launch_host_word(uint32_t * word, uint32_t tag, hipStream_t s) {
+    k_host_word<<<1, 1, 0, s>>>(word, tag);
+    CHECK_LAUNCH();
+    return hipSuccess;
+}
+
 __global__ void k_zero_i32(int32_t * p, int64_t n) {
     for (int64_t i = (int64_t) blockIdx.x * blockDim.x + threadIdx.x; i < n; i += (int64_t) gridDim.x * blockDim.x)
         p[i] = 0;

@@ -226,6 +226,8 @@ int chain_occupancy(int fmt, int ring, size_t lds);
 hipError_t launch_npu_stage(int fmt, const uint8_t * src, int64_t sstride, const NpuGeom & g, const int32_t * rowmap,
                             int64_t N, int64_t K, uint8_t * dst, int64_t dstride, int64_t E, hipStream_t s);
 // p[0, n) = 0 by a kernel on stream s (a graph node under capture, unlike a memset)
+// *word = tag (host memory the GPU sees), after all earlier work on s
+hipError_t launch_host_word(uint32_t * word, uint32_t tag, hipStream_t s);
 hipError_t launch_zero_i32(int32_t * p, int64_t n, hipStream_t s);
 // y[t] = sum_j w[t][j] o[inv[t k + j]] (o bf16 rows, fp32 sum)
 hipError_t launch_moe_combine(const uint16_t * o, const int32_t * inv, const float * w, int64_t T, int k, int64_t N,

@@ -14,12 +14,14 @@ from ._lib import check, require_gpu
 
 
 def _stream():
+    """the handle of torch's current stream (0.3 us; through a torch.cuda.Stream object 3.2 us of the
+    8.6 that issuing a matrix product took)"""
     import torch
-    return C.c_void_p(torch.cuda.current_stream().cuda_stream)
+    return torch._C._cuda_getCurrentRawStream(torch.cuda.current_device())
 
 
 def _ptr(t):
-    return C.c_void_p(t.data_ptr())
+    return t.data_ptr()
 
 
 def _np_ptr(a):

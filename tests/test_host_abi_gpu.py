@@ -326,3 +326,27 @@ def test_ffn_run_reports_a_timed_out_wait(L, monkeypatch):
                 assert b"MoE decode's wait for its act rows gave up" in L.onpu_last_error()
     finally:
         L.onpu_ffn_free(f)
+
+
+@pytest.mark.parametrize("N,K,M", [(40, 128, 1), (8192, 256, 8), (8200, 256, 8), (64, 8192, 8), (64, 8320, 8),
+                                   (1000, 4096, 96)])
+def test_dense_mv_pinned_range(gpu, N, K, M):
+    """onpu_dense_mv with x and y through pinned memory, up to 256 KiB each, and past it through the
+    device staging: two inputs in turn, and again after onpu_release_scratch"""
+    import ctypes as C
+    from opennpu_amd import synthetic as syn
+    from opennpu_amd.device import QMatrix
+    fmt, F = orc.FMT_G128S, C.POINTER(C.c_float)
+    st = syn.weights(fmt, N, K, 3)
+    q = QMatrix(N, K, fmt, st)
+    try:
+        for seed in (1, 2, 1):
+            x = np.random.default_rng(seed).standard_normal((M, K)).astype(np.float32)
+            y = np.full((M, N), np.nan, np.float32)
+            gpu.onpu_dense_mv(q.h, x.ctypes.data_as(F), M, y.ctypes.data_as(F))
+            ref = orc.qmm(fmt, st, N, K, xbits(x), bf16w=M > 32)
+            assert np.abs(y - ref).max() <= 1e-4 * np.abs(ref).max()
+            if seed == 2:
+                gpu.onpu_release_scratch()
+    finally:
+        q.free()
