@@ -693,11 +693,12 @@ bool rows_take_gemv(int64_t M, int64_t N, int64_t K) {
 
 // mv_core's choice for M rows: the decode GEMV (path 0), k_qgemm with mb A blocks of 16 rows and ntw
 // weight tiles per wave, in S ranges of kbs K blocks (path 1), or k_qgemm_sk (path 2); wgs: k_qgemm's
-// workgroups per K range; deep: 16-row tiles with the weights two blocks ahead
-struct MvPlan { int path, mb, ntw; int64_t S, kbs, wgs; int deep; };
+// workgroups per K range; deep: 16-row tiles with the weights two blocks ahead; kg: K ranges that one
+// workgroup takes
+struct MvPlan { int path, mb, ntw; int64_t S, kbs, wgs; int deep, kg; };
 
 MvPlan plan_mv(int fmt, int64_t N, int64_t K, int64_t NT, int64_t KB, int64_t M, int cus) {
-    MvPlan p{0, 8, 2, 1, KB, 0, 0};
+    MvPlan p{0, 8, 2, 1, KB, 0, 0, 1};
     if (rows_take_gemv(M, N, K)) return p;
     int cfg = 0;
     int64_t grid = 0;
@@ -724,6 +725,7 @@ MvPlan plan_mv(int fmt, int64_t N, int64_t K, int64_t NT, int64_t KB, int64_t M,
     if (p.ntw != 2) p.mb = 8;
     // the kernel addresses X with 32-bit buffer offsets: launches of at most 2^31 bytes of X rows
     const int64_t rows_max = std::max<int64_t>(128, (((int64_t) 1 << 31) - 1) / (K * 2) / 128 * 128);
+    const bool dtile = p.mb == 1 || (p.mb == 2 && fmt == ONPU_G128S && N * K >= 100000000);   // see p.deep
     // split-K when the tiles leave CUs without work: S K ranges, S x the workgroups (two per CU,
     // at least 4 K blocks each), fp32 partials in the split-K workspace, then their sum. A sweep of
     // S over 1-16 (65-512 rows, seven shapes; 1-64 rows, thirteen shapes and formats) put this rule
@@ -732,6 +734,24 @@ MvPlan plan_mv(int fmt, int64_t N, int64_t K, int64_t NT, int64_t KB, int64_t M,
     if (M <= rows_max) {
         const int es = env_int("ONPU_GEMM_SPLIT", 0);
         int64_t S = es >= 1 ? es : std::min<int64_t>(KB / 4, 2 * (int64_t) cus / p.wgs);
+        // K groups of one workgroup (k_qgemm's KG, one workgroup per CU): the partials are planes, not
+        // ranges, or go with their sum launch. Taken where no CU gets more K blocks than with single
+        // groups (for up to 64 rows a fifth more, as the partials weigh more). us per call, one group ->
+        // KG, 3 matrices in turn: 24576 x 4096 at 32 rows q4nx 24.2 -> 20.5, 4096 x 14336 at 24 / 96 14.3 /
+        // 30.5 -> 13.4 / 28.5, 14336 x 4096 at 30 / 48 / 100 15.9 / 20.2 / 32.2 -> 14.8 / 18.3 / 30.6, 4096 x
+        // 4096 at 200 28.6 -> 25.9, 12345 x 2048 at 70 26.6 -> 21.8, 9000 x 1056 at 150 23.7 -> 18.6. With more
+        // blocks per CU slower: 1500 x 4096 at 1000 (8 against 7 in two groups) 32.7 -> 34.6, 2000 x 2048 at
+        // 128 (8 against 4) 17.2 -> 19.3; with two such workgroups on a CU too: 3000 x 8192 at 300 38.9 ->
+        // 61.5. (g128s 32-row tiles of larger matrices keep their weights two blocks ahead instead.)
+        if (S > 1 && p.ntw == 2 && p.mb >= 2 && !(p.mb == 2 && dtile)) {
+            const int kg = p.mb == 8 ? 2 : 4;
+            const int64_t g = es >= 1 ? S : std::min<int64_t>(KB / 4, (int64_t) cus / p.wgs * kg), planes = (g + kg - 1) / kg;
+            const int64_t one = (S * p.wgs + cus - 1) / cus * ((KB + S - 1) / S), grp = g > 1 ? kg * ((KB + g - 1) / g) : KB * kg;
+            if (g > 1 && planes * p.wgs <= cus && (p.mb == 8 ? grp <= one : 5 * grp <= 6 * one)) {
+                p.kg = kg;
+                S = g;
+            }
+        }
         S = std::max<int64_t>(1, std::min<int64_t>(S, KB));
         while (S > 1 && (size_t) (S * M * N * 4) > gsk_part_bytes(cus)) S--;
         if (S > 1) {
@@ -744,7 +764,6 @@ MvPlan plan_mv(int fmt, int64_t N, int64_t K, int64_t NT, int64_t KB, int64_t M,
     // matrices (57344 x 8192 at 17-32 rows 81-84 -> 74-80 us, 24576 x 4096 24.1-25.3 -> 22.5-24.0;
     // the per-32 formats and matrices below 1e8 weights measured 1-7 % slower there)
     const int ed = env_int("ONPU_GEMM_DEEP", -1);
-    const bool dtile = p.mb == 1 || (p.mb == 2 && fmt == ONPU_G128S && N * K >= 100000000);
     p.deep = p.ntw == 2 && p.mb <= 2 && (ed >= 0 ? ed != 0 : dtile && p.S * p.wgs <= 2 * (int64_t) cus);
     return p;
 }
@@ -771,13 +790,14 @@ hipError_t mv_core(Mat4 * m, int64_t e, const uint16_t * x, int64_t M, void * y,
     if (p.S > 1) {
         GArgs a{};
         int32_t * sync = nullptr, * ctl = nullptr;
-        hipError_t e = gsk_workspace(s, 0, &a.ws, &sync, &ctl);
+        const int64_t planes = (p.S + p.kg - 1) / p.kg;
+        hipError_t e = planes > 1 ? gsk_workspace(s, 0, &a.ws, &sync, &ctl) : hipSuccess;
         if (e != hipSuccess) return e;
         a.W = W; a.NT = m->g.NT; a.KB = m->g.KB; a.N = m->N; a.K = m->K; a.M = M;
-        a.x = x; a.ldx = m->K; a.ldy = m->N; a.yf32 = 1; a.y = a.ws;
-        a.splits = (int) p.S; a.kbs = p.kbs; a.deep = p.deep;
-        if ((e = launch_qgemm(m->fmt, a, p.ntw, p.mb, s)) != hipSuccess) return e;
-        return launch_gemm_split_sum(a.ws, (int) p.S, M, m->N, y, m->N, yf32, s);
+        a.x = x; a.ldx = m->K; a.ldy = m->N; a.yf32 = planes > 1 ? 1 : yf32; a.y = planes > 1 ? a.ws : y;
+        a.splits = (int) p.S; a.kbs = p.kbs; a.deep = p.deep; a.kgroups = p.kg;
+        if ((e = launch_qgemm(m->fmt, a, p.ntw, p.mb, s)) != hipSuccess || planes == 1) return e;
+        return launch_gemm_split_sum(a.ws, (int) planes, M, m->N, y, m->N, yf32, s);
     }
     const int64_t rows_max = std::max<int64_t>(128, (((int64_t) 1 << 31) - 1) / (m->K * 2) / 128 * 128);
     for (int64_t r0 = 0; r0 < M; r0 += rows_max) {

@@ -37,7 +37,16 @@ hipError_t FN(qgemv)(int epi, const QArgs & a, int mb, int rt, int nb, int xl, d
 
 hipError_t FN(qgemm)(const GArgs & a, int ntw, int mb, hipStream_t s) {
     const int64_t gm = (a.M + 16 * mb - 1) / (16 * mb), gn = (a.NT + 4 * ntw - 1) / (4 * ntw);
-    const dim3 grid((unsigned) (gm * gn * (a.splits > 1 ? a.splits : 1)));
+    const int64_t planes = a.splits > 1 ? (a.splits + a.kgroups - 1) / a.kgroups : 1;
+    const dim3 grid((unsigned) (gm * gn * planes));
+    if (a.splits > 1 && a.kgroups > 1) {
+        if (ntw != 2) return hipErrorInvalidValue;
+        if (mb == 2 && a.kgroups == 4) k_qgemm<F, 2, 2, false, false, 4><<<grid, 1024, 0, s>>>(a);
+        else if (mb == 4 && a.kgroups == 4) k_qgemm<F, 2, 4, false, false, 4><<<grid, 1024, 0, s>>>(a);
+        else if (mb == 8 && a.kgroups == 2) k_qgemm<F, 2, 8, false, false, 2><<<grid, 512, 0, s>>>(a);
+        else return hipErrorInvalidValue;
+        return hipGetLastError();
+    }
     if (a.akeys) {                            // argmax keys: one row tile, no split (host checked)
         if (mb == 1 && a.deep) k_qgemm<F, 2, 1, true, true><<<grid, 256, 0, s>>>(a);
         else if (mb == 1) k_qgemm<F, 2, 1, true><<<grid, 256, 0, s>>>(a);

@@ -1074,13 +1074,18 @@ DEV void gemm_load_w(const __amdgpu_buffer_rsrc_t (&wrs)[NTW], int64_t b, int la
 // each row over its columns in a.akeys[m][N block] (argmax_key: larger value, then lower column)
 // DEEP (16- and 32-row tiles): weights two blocks ahead (three register sets), for grids of at
 // most two workgroups per CU, where one block in flight per workgroup leaves the memory idle
-template <int FMT, int NTW, int MB, bool AK = false, bool DEEP = false>
-__global__ __launch_bounds__(256, MB == 8 ? 2 : 4) void k_qgemm(GArgs a) {
-    __shared__ u32x4 xs0[MB * 4 * 64], xs1[MB * 4 * 64];   // 2 x MB x 4 KiB
+// KG: K groups of 4 waves per workgroup: group g takes K range KG sp + g (its own X buffers), the groups'
+// sums meet in LDS, and the workgroup stores one plane of partials (Y itself if it is the only one). What it
+// saves is the planes: 4096 x 14336 at 96 rows wrote and read 25 MB of them for 29 MB of weights (30.5 -> 28.5
+// us), 24576 x 4096 at 32 rows 6.3 MB and a second launch (24.2 -> 20.5 us); plan_mv has the rule
+template <int FMT, int NTW, int MB, bool AK = false, bool DEEP = false, int KG = 1>
+__global__ __launch_bounds__(256 * KG, KG > 1 ? 1 : (MB == 8 ? 2 : 4)) void k_qgemm(GArgs a) {
+    __shared__ u32x4 xs0_[KG * MB * 4 * 64], xs1_[KG * MB * 4 * 64];   // 2 x MB x 4 KiB per K group
     constexpr int MT = 16 * MB;                           // rows of the workgroup tile
     constexpr int BLK = 1024 + 16 * (128 / (FMT == ONPU_G128S ? 128 : 32)) * 2 * (FMT == ONPU_Q4NX ? 2 : 1);
-    const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6), r = lane & 15;
-    const int q = lane >> 4;
+    const int tid = threadIdx.x, lane = tid & 63, r = lane & 15, q = lane >> 4;
+    const int wv = __builtin_amdgcn_readfirstlane(tid >> 6), wave = wv & 3, kg = KG > 1 ? wv >> 2 : 0;
+    u32x4 * const xs0 = xs0_ + kg * (MB * 4 * 64), * const xs1 = xs1_ + kg * (MB * 4 * 64);
     const int64_t nwg = (int64_t) gridDim.x, wg = blockIdx.x;
     int64_t lid = wg;
     if (nwg % 8 == 0) lid = (wg % 8) * (nwg / 8) + wg / 8;
@@ -1097,11 +1102,14 @@ __global__ __launch_bounds__(256, MB == 8 ? 2 : 4) void k_qgemm(GArgs a) {
     if (a.splits > 1) {
         const int64_t sp = lid / (gm * gn);
         lid -= sp * (gm * gn);
-        kb0 = sp * a.kbs;
+        kb0 = (sp * KG + kg) * a.kbs;
+        if (KG > 1 && kb0 > a.KB) kb0 = a.KB;                // no range left for this group
         kb1 = kb0 + a.kbs < a.KB ? kb0 + a.kbs : a.KB;
-        yo = a.ws + sp * a.M * a.N;
-        ldy = a.N;
-        yf32 = 1;
+        if (a.splits > KG) {
+            yo = a.ws + sp * a.M * a.N;
+            ldy = a.N;
+            yf32 = 1;
+        }
     }
     const int64_t grp = lid / (GMS * gn), in = lid % (GMS * gn);
     const int64_t gms = gm - grp * GMS < GMS ? gm - grp * GMS : GMS;       // M tiles in this group
@@ -1192,6 +1200,56 @@ __global__ __launch_bounds__(256, MB == 8 ? 2 : 4) void k_qgemm(GArgs a) {
             __syncthreads();
         }
         __builtin_amdgcn_s_waitcnt(0x0f70);               // vmcnt(0): no load still writes LDS
+    } else if constexpr (KG > 1) {
+        // the stages of all groups in step (the barriers are the workgroup's); a group past its blocks
+        // only waits
+        const int nb = (int) (kb1 - kb0), ns = (int) a.kbs;
+        auto load = [&](int i, u32x4 * xsb, u32x4 (&w)[NTW], GPar<FMT> (&p)[NTW]) {
+            if (i >= nb) return;
+            gemm_load_x(xr, xo, kb0 + i, ktail && kb0 + i + 1 == a.KB, a.K, wave, q, xsb);
+            gemm_load_w<FMT, NTW>(wrs, kb0 + i, lane, r, w, p);
+        };
+        load(0, xs0, wa, pa);
+        __builtin_amdgcn_s_waitcnt(0x0f70);
+        __syncthreads();
+        for (int i = 0; i < ns; i += 2) {
+            load(i + 1, xs1, wb, pb);
+            if (i < nb) blk(xs0, wa, pa);
+            __builtin_amdgcn_s_waitcnt(0x0f70);
+            __syncthreads();
+            load(i + 2, xs0, wa, pa);
+            if (i + 1 < nb) blk(xs1, wb, pb);
+            __builtin_amdgcn_s_waitcnt(0x0f70);
+            __syncthreads();
+        }
+        // the groups' sums: row blocks below MB / 2 through xs0_, the others through xs1_ ([KG][MB / 2][4
+        // waves][NTW][4][64] floats each); group g adds and stores the (row block, tile) pairs g, g + KG, ...
+        constexpr int PW = NTW * 4 * 64, PG = MB / 2 * 4 * PW;
+        auto red = [&](int g, int mb) {
+            return (float *) (mb < MB / 2 ? xs0_ : xs1_) + g * PG + (mb % (MB / 2) * 4 + wave) * PW + lane;
+        };
+#pragma unroll
+        for (int mb = 0; mb < MB; mb++)
+#pragma unroll
+            for (int i = 0; i < NTW; i++)
+#pragma unroll
+                for (int v = 0; v < 4; v++) red(kg, mb)[(i * 4 + v) * 64] = acc[mb][i][v];
+        __syncthreads();
+#pragma unroll
+        for (int u = 0; u < MB * NTW / KG; u++) {
+            const int mb = (u * KG + kg) / NTW, i = (u * KG + kg) % NTW;
+            const int64_t n = 16 * (t0 + i) + r;
+            if (i >= nt_ok || n >= a.N) continue;
+#pragma unroll
+            for (int v = 0; v < 4; v++) {
+                const int64_t m = m0 + 16 * mb + 4 * q + v;
+                float sum = red(0, mb)[(i * 4 + v) * 64];
+#pragma unroll
+                for (int g = 1; g < KG; g++) sum += red(g, mb)[(i * 4 + v) * 64];
+                if (m < a.M) store_out(yo, yf32, m * ldy + n, sum);
+            }
+        }
+        return;
     } else {
     gemm_load_x(xr, xo, kb0, ktail && kb0 + 1 == a.KB, a.K, wave, q, xs0);
     gemm_load_w<FMT, NTW>(wrs, kb0, lane, r, wa, pa);

@@ -64,6 +64,8 @@ struct GArgs {
     // adds the splits in order into Y
     int splits;
     int64_t kbs;
+    int kgroups;              // K ranges that one workgroup takes and sums (1, or 2 / 4 as built): planes of
+                              // partials ceil(splits / kgroups), none with one
     // k_qgemm, one row tile and no split: also each workgroup's argmax key per row, akeys[m][N block]
     uint64_t * akeys;
     int deep;                 // k_qgemm 16-row tiles: weights two blocks ahead

@@ -232,6 +232,42 @@ def test_gemm_split_k(gpu, fmt, M, N, K, mb, monkeypatch):
     check_f32_out(yf, orc.qmm(fmt, st, N, K, xb[rows], bf16w=True), what=f"split-K fmt {fmt} fp32 rows")
 
 
+@pytest.mark.parametrize("fmt", FMTS)
+@pytest.mark.parametrize("M,N,K,S", [(24, 24576, 1024, 2), (30, 14300, 2048, 4), (40, 14000, 2048, 3), (64, 24576, 1024, 2),
+                                     (70, 12345, 1024, 2), (96, 4096, 1920, 3), (150, 9000, 1152, 2)])
+def test_gemm_k_groups(gpu, fmt, M, N, K, S, monkeypatch):
+    """GEMMs whose workgroups take several K ranges (2 or 4 groups of 4 waves), forced to S ranges: fewer
+    ranges than groups, one plane stored as Y and several, a last range shorter than the others, odd N:
+    a column slice and three rows against the oracle, and the unsplit kernel to fp32 summation order"""
+    import torch
+    from opennpu_amd.device import QMatrix
+    if fmt != orc.FMT_G128S:
+        K -= 32
+    st, xb = syn.weights(fmt, N, K, 61), syn.activations(M, K, 62)
+    q = QMatrix(N, K, fmt, st)
+    try:
+        x = to_torch_bf16(xb).reshape(M, K)
+        yd = q.mv(x, f32=True)
+        monkeypatch.setenv("ONPU_GEMM_SPLIT", str(S))
+        ys = q.mv(x, f32=True)
+        yb = q.mv(x)
+        monkeypatch.setenv("ONPU_GEMM_SPLIT", "1")
+        y1 = q.mv(x, f32=True)
+        monkeypatch.delenv("ONPU_GEMM_SPLIT")
+        torch.cuda.synchronize()
+        for y in (yd, ys):
+            # sums of K products in another order: 1e-5 of the largest, as test_gemm_split_k
+            assert ((y - y1).abs().max() / y1.abs().max()).item() <= 1e-5
+        assert torch.equal(yb, ys.to(torch.bfloat16))
+        rows = [0, M // 2, M - 1]
+        yc, yr = from_torch(ys[:, N - 200:]), from_torch(ys[rows])
+    finally:
+        q.free()
+    bw = not gemm_exact(fmt, M)
+    check_f32_out(yc, orc.qmm(fmt, st, N, K, xb, N - 200, N, bf16w=bw), what="columns")
+    check_f32_out(yr, orc.qmm(fmt, st, N, K, xb[rows], bf16w=bw), what="rows")
+
+
 def test_gemm_split_k_under_capture(gpu):
     """split-K GEMMs recorded in a graph (their partials in the capture's own workspace) at 96, 40
     and 16 rows (128-, 64- and 16-row tiles, the last with the weights two blocks ahead), and the
