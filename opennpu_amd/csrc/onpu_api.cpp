@@ -131,11 +131,15 @@ struct HostPin {
     float * x() const { return (float *) p; }
     float * y() const { return (float *) (p + HP_BYTES); }
     uint32_t * word() const { return (uint32_t *) (p + 2 * HP_BYTES); }
-    bool ready() {
-        if (!p && hipHostMalloc((void **) &p, 2 * HP_BYTES + 64, hipHostMallocCoherent) != hipSuccess) {
+    bool ready() {                           // (relaxed capture mode: another thread may be capturing)
+        if (p) return true;
+        hipStreamCaptureMode mode = hipStreamCaptureModeRelaxed;
+        if (hipThreadExchangeStreamCaptureMode(&mode) != hipSuccess) return false;
+        if (hipHostMalloc((void **) &p, 2 * HP_BYTES + 64, hipHostMallocCoherent) != hipSuccess) {
             (void) hipGetLastError();
             p = nullptr;
         }
+        (void) hipThreadExchangeStreamCaptureMode(&mode);
         return p != nullptr;
     }
     void release() {
