@@ -39,17 +39,7 @@ struct AttnArgs {
     int Hq, D, Hkv, rep, ngrp, C, nch;
 };
 
-template <typename KV> __device__ __forceinline__ void load8(const KV * p, float (&v)[8]);
-template <> __device__ __forceinline__ void load8<uint16_t>(const uint16_t * p, float (&v)[8]) {
-    const uint4 u = *(const uint4 *) p;
-    const uint32_t w[4] = {u.x, u.y, u.z, u.w};
-#pragma unroll
-    for (int i = 0; i < 4; i++) {
-        v[2 * i] = __uint_as_float(w[i] << 16);
-        v[2 * i + 1] = __uint_as_float(w[i] & 0xffff0000u);
-    }
-}
-template <> __device__ __forceinline__ void load8<float>(const float * p, float (&v)[8]) {
+__device__ __forceinline__ void load8(const float * p, float (&v)[8]) {
     const float4 a = *(const float4 *) p, b = *(const float4 *) (p + 4);
     v[0] = a.x; v[1] = a.y; v[2] = a.z; v[3] = a.w;
     v[4] = b.x; v[5] = b.y; v[6] = b.z; v[7] = b.w;
@@ -80,7 +70,7 @@ __device__ __forceinline__ float wave_sum(float v) {
 }
 
 // LDS: P [HG][C], red [AW][HG][D], wmax / wsum [AW][HG], qs [HG][D]
-template <typename KV, int LPR, int HG>
+template <int LPR, int HG>
 __global__ __launch_bounds__(AT) void k_attn_part(AttnArgs a) {
     constexpr int RPW = 64 / LPR, RIT = AW * RPW * AU;          // row slots per wave; rows per pass
     extern __shared__ __align__(16) float lds[];
@@ -91,8 +81,8 @@ __global__ __launch_bounds__(AT) void k_attn_part(AttnArgs a) {
     const int64_t j0 = (int64_t) c * C;
     const int rows = (int) (a.S - j0 < C ? a.S - j0 : C);
     // lanes past D read column 0 (their values meet zero q and are never stored)
-    const KV * Kg = (const KV *) a.K + (int64_t) g * a.hs + j0 * a.rs + 8 * (dl ? li : 0);
-    const KV * Vg = (const KV *) a.V + (int64_t) g * a.hs + j0 * a.rs + 8 * (dl ? li : 0);
+    const float * Kg = (const float *) a.K + (int64_t) g * a.hs + j0 * a.rs + 8 * (dl ? li : 0);
+    const float * Vg = (const float *) a.V + (int64_t) g * a.hs + j0 * a.rs + 8 * (dl ? li : 0);
     // q of the group's heads: coalesced 16-byte loads (0 past rep), stored to LDS after the first
     // pass's K loads are issued; the barrier then waits for LDS only (a __syncthreads would also
     // wait for the K loads)
@@ -104,13 +94,13 @@ __global__ __launch_bounds__(AT) void k_attn_part(AttnArgs a) {
     // Row of (pass r0, step u, wave, slot): consecutive slots and waves take consecutive rows, so one
     // wave instruction reads RPW consecutive rows.
     float kv[AU][8];
-    auto issue = [&](const KV * base, int r0) {
+    auto issue = [&](const float * base, int r0) {
 #pragma unroll
         for (int u = 0; u < AU; u++) {
             // rows past the chunk re-read its last row: their scores are not stored, their V rows
             // not accumulated
             const int row = r0 + (u * AW + wave) * RPW + slot;
-            load8<KV>(base + (int64_t) (row < rows ? row : rows - 1) * a.rs, kv[u]);
+            load8(base + (int64_t) (row < rows ? row : rows - 1) * a.rs, kv[u]);
         }
     };
     issue(Kg, 0);
@@ -638,7 +628,7 @@ hipError_t run_attn(const AttnArgs & a, const AttnPlan & p, hipStream_t s) {
                            std::max<size_t>(sizeof(float) * MW * HG * a.D, 1024 * (size_t) NS * ((HG + 3) / 4));
         k_attn_mfma<NS, HG, KT><<<grid, MT, lds, s>>>(a);
     } else {
-        k_attn_part<float, 4 * NS, HG><<<grid, AT, attn_lds(p, a.D), s>>>(a);
+        k_attn_part<4 * NS, HG><<<grid, AT, attn_lds(p, a.D), s>>>(a);
     }
     hipError_t e = hipGetLastError();
     if (e != hipSuccess || (BF && a.nch == 1)) return e;
