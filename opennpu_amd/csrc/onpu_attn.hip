@@ -140,7 +140,8 @@ __global__ __launch_bounds__(AT) void k_attn_part(AttnArgs a) {
     issue(Vg, 0);                           // phase 2's first V loads fly during the softmax
     __builtin_amdgcn_s_waitcnt(0xc07f);
     __builtin_amdgcn_s_barrier();
-    // chunk max and exp-sum per head (a chunk whose rows are all -inf keeps p = 0)
+    // chunk max and exp-sum per head (a chunk whose rows are all -inf gets
+    // p = e^(-inf - 0) = 0; a NaN score, which the maximum skips, p = NaN)
 #pragma unroll
     for (int h = 0; h < HG; h++) {
         float mx = -__builtin_inff();
@@ -155,9 +156,10 @@ __global__ __launch_bounds__(AT) void k_attn_part(AttnArgs a) {
         float mx = wmax[h];
 #pragma unroll
         for (int w = 1; w < AW; w++) mx = fmaxf(mx, wmax[w * HG + h]);
+        const float base = mx == -__builtin_inff() ? 0.f : mx;
         float l = 0.f;
         for (int r = t; r < rows; r += AT) {
-            const float p = mx == -__builtin_inff() ? 0.f : expf(P[h * C + r] - mx);
+            const float p = expf(P[h * C + r] - base);
             P[h * C + r] = p;
             l += p;
         }
@@ -398,9 +400,10 @@ __global__ __launch_bounds__(MT, 2) void k_attn_mfma(AttnArgs a) {
             up = up || m[h4] != mx;
             m[h4] = mx;
             l[h4] *= al[h4];
+            const float base = mx == -__builtin_inff() ? 0.f : mx;           // -inf rows alone: p = 0; NaN: p = NaN
 #pragma unroll
             for (int t = 0; t < KT; t++) {
-                const float p = mx == -__builtin_inff() ? 0.f : expf(sc[t][h4] - mx);
+                const float p = expf(sc[t][h4] - base);
                 l[h4] += p;
                 if (4 * h4 + quad < HG) P[(16 * t + key) * HG + 4 * h4 + quad] = p;
             }

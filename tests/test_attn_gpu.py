@@ -108,6 +108,39 @@ def test_attn_step_dev_tails(gpu, Hq, Hkv, D, S):
     assert err <= TOL, err
 
 
+@pytest.mark.parametrize("kv", ["bf16", "f32"])
+@pytest.mark.parametrize("Hq,Hkv,D,S", [(8, 2, 64, 300), (32, 8, 128, 700), (6, 3, 256, 2900), (16, 1, 128, 5000)])
+def test_attn_step_dev_nan_scores(gpu, kv, Hq, Hkv, D, S):
+    """a NaN in K, alone among masked rows of its step of 16, of its wave's pass and of its chunk: every
+    output of that kv head's query heads is NaN, as in the reference (the sum of the weights is), and
+    the other heads' are as without it; the same with no finite score at all"""
+    import torch
+    from opennpu_amd.device import attn_step
+    rng = np.random.default_rng(S + D)
+    q, K, V, _, sk = _case(rng, Hq, Hkv, D, S, S, kv, False, True)
+    up = orc.bf2f if kv == "bf16" else (lambda a: a)
+    down = orc.f2bf_np if kv == "bf16" else (lambda a: a)
+    Kf = up(K).reshape(Hkv, S, D).copy()
+    row, gh = S - 60, Hkv - 1
+    Kf[gh, row, 3] = np.nan
+    K, V = down(Kf).reshape(Hkv, S, D), V.reshape(Hkv, S, D)
+    to = (lambda a: torch.from_numpy(np.ascontiguousarray(a).view(np.int16)).view(torch.bfloat16).cuda()) if kv == "bf16" \
+        else (lambda a: torch.from_numpy(np.ascontiguousarray(a)).cuda())
+    for first in (20, 0):                                    # finite rows: [0, 20), or none
+        mask = np.full(S, -np.inf, np.float32)
+        mask[:first] = 0.0
+        mask[row] = 0.0
+        with np.errstate(invalid="ignore"):
+            ref = orc.attn_step(q, K, V, mask, sk)
+        bad = np.repeat(np.arange(Hkv) == gh, Hq // Hkv)
+        assert np.isnan(ref[bad]).all() and np.isfinite(ref[~bad]).all()
+        out = attn_step(torch.from_numpy(q).cuda(), to(K), to(V), torch.from_numpy(mask).cuda(),
+                        torch.from_numpy(sk).cuda()).cpu().numpy()
+        assert np.array_equal(np.isnan(out), np.isnan(ref)), first
+        if not bad.all():
+            assert np.abs(out[~bad] - ref[~bad]).max() <= TOL * max(np.abs(ref[~bad]).max(), 1e-30)
+
+
 def test_attn_step_dev_argument_errors(gpu):
     """rejected on the host, nothing launched: Hq not a multiple of Hkv, D not a multiple of 8,
     more than 16 query heads per kv head, a short workspace"""
