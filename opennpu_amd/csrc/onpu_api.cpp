@@ -697,8 +697,9 @@ bool rows_take_gemv(int64_t M, int64_t N, int64_t K) {
 
 // mv_core's choice for M rows: the decode GEMV (path 0), k_qgemm with mb A blocks of 16 rows and ntw
 // weight tiles per wave, in S ranges of kbs K blocks (path 1), or k_qgemm_sk (path 2); wgs: k_qgemm's
-// workgroups per K range; deep: 16-row tiles with the weights two blocks ahead; kg: K ranges that one
-// workgroup takes
+// workgroups per K range, or per kg ranges: kg ranges go to one workgroup, which sums them, so that the
+// launch has ceil(S / kg) wgs workgroups and leaves as many planes of partials; deep: 16- and 32-row tiles
+// with the weights two blocks ahead
 struct MvPlan { int path, mb, ntw; int64_t S, kbs, wgs; int deep, kg; };
 
 MvPlan plan_mv(int fmt, int64_t N, int64_t K, int64_t NT, int64_t KB, int64_t M, int cus) {
@@ -762,6 +763,7 @@ MvPlan plan_mv(int fmt, int64_t N, int64_t K, int64_t NT, int64_t KB, int64_t M,
             p.kbs = (KB + S - 1) / S;
             p.S = (KB + p.kbs - 1) / p.kbs;
         }
+        if (p.S == 1) p.kg = 1;
     }
     // weights two blocks ahead with at most two workgroups per CU (one block in flight per
     // workgroup leaves the memory idle there): 16-row tiles, and g128s 32-row tiles of larger
@@ -1104,8 +1106,6 @@ void onpu_stats(int64_t * calls, double * wait_s) {
 // every (tiles, kc) is served: the HIP kernels take any shape
 int onpu_has_shape(int, int, int) { return device().ok; }
 
-// the GEMV launch plan for an [N][K] matrix of fmt at M rows over `slots` (host only, no GPU):
-// out = mb, rt, nb, xl, tw, kw, bpw, gx, built (1 if that kernel variant exists), max waves
 void onpu_plan_mv(int fmt, int64_t N, int64_t K, int64_t M, int64_t * out) {
     const Tiled g = tiled_geom(fmt, N, K);
     const MvPlan p = plan_mv(fmt, N, K, g.NT, g.KB, M, device().cus > 0 ? device().cus : 256);
@@ -1113,6 +1113,13 @@ void onpu_plan_mv(int fmt, int64_t N, int64_t K, int64_t M, int64_t * out) {
     for (int i = 0; i < 7; i++) out[i] = v[i];
 }
 
+int onpu_plan_mv_groups(int fmt, int64_t N, int64_t K, int64_t M) {
+    const Tiled g = tiled_geom(fmt, N, K);
+    return plan_mv(fmt, N, K, g.NT, g.KB, M, device().cus > 0 ? device().cus : 256).kg;
+}
+
+// the GEMV launch plan for an [N][K] matrix of fmt at M rows over `slots` (host only, no GPU):
+// out = mb, rt, nb, xl, tw, kw, bpw, gx, built (1 if that kernel variant exists), max waves
 void onpu_plan_gemv(int fmt, int64_t N, int64_t K, int M, int64_t slots, int epi, int64_t * out) {
     const Tiled g = tiled_geom(fmt, N, K);
     const Plan p = epi == EPI_SLOTSUM_ ? plan_slotsum(g.KB, (int) slots) : plan_gemv(fmt, g.NT, g.KB, M, slots, epi);

@@ -139,6 +139,33 @@ def test_mv_plans():
     assert {(0, 0, 0), (1, 1, 0), (1, 1, 1), (1, 2, 0), (1, 2, 1), (1, 4, 0), (1, 8, 0), (2, 0, 0)} <= seen, seen
 
 
+def test_mv_plan_groups():
+    """onpu_plan_mv_groups, the K ranges that one workgroup of the planned GEMM takes: 4 (tiles of 32 or
+    64 rows) or 2 (128 rows) only with several ranges, at most one workgroup per CU over all planes of
+    partials, no fewer than the 4 K blocks of a range each; and what 24576 x 4096 at 32 rows (one
+    plane, no sum) and 4096 x 14336 at 96 rows (8 planes) run"""
+    L = _lib.lib()
+    o = (C.c_int64 * 7)()
+    seen = set()
+    for fmt in range(4):
+        for N in (64, 1000, 4096, 9000, 14336, 24576, 57344):
+            for K in (512, 1024, 4096, 8192, 14336):
+                for M in (1, 8, 16, 24, 32, 48, 64, 96, 150, 256, 512, 2048):
+                    L.onpu_plan_mv(fmt, N, K, M, o)
+                    path, mb, ntw, S, kbs, wgs, deep = tuple(o)
+                    g = L.onpu_plan_mv_groups(fmt, N, K, M)
+                    seen.add((mb, g) if path == 1 else path)
+                    assert g in (1, 2, 4), (fmt, N, K, M)
+                    if g > 1:
+                        assert path == 1 and S > 1 and ntw == 2 and not deep and kbs >= 4, (fmt, N, K, M, tuple(o))
+                        assert g == (2 if mb == 8 else 4) and mb >= 2 and -(-S // g) * wgs <= 256, (fmt, N, K, M, g, tuple(o))
+    assert {(2, 4), (4, 4), (8, 2), (2, 1), (4, 1), (8, 1), (1, 1), 0, 2} <= seen, seen
+    L.onpu_plan_mv(0, 24576, 4096, 32, o)
+    assert (o[3], o[5], L.onpu_plan_mv_groups(0, 24576, 4096, 32)) == (4, 192, 4)
+    L.onpu_plan_mv(2, 4096, 14336, 96, o)
+    assert (o[3], o[5], L.onpu_plan_mv_groups(2, 4096, 14336, 96)) == (16, 32, 2)
+
+
 @pytest.mark.parametrize("fmt", [0, 1, 2, 3])
 def test_argmax_epilogue_plans_sum_like_the_store(fmt):
     """the argmax epilogue's GEMV plan (onpu_dense_argmax_dev) and the plain store's (the no-alloc
