@@ -730,6 +730,7 @@ MvPlan plan_mv(int fmt, int64_t N, int64_t K, int64_t NT, int64_t KB, int64_t M,
     if (p.ntw != 2) p.mb = 8;
     // the kernel addresses X with 32-bit buffer offsets: launches of at most 2^31 bytes of X rows
     const int64_t rows_max = std::max<int64_t>(128, (((int64_t) 1 << 31) - 1) / (K * 2) / 128 * 128);
+    const int ed = env_int("ONPU_GEMM_DEEP", -1);
     const bool dtile = p.mb == 1 || (p.mb == 2 && fmt == ONPU_G128S && N * K >= 100000000);   // see p.deep
     // split-K when the tiles leave CUs without work: S K ranges, S x the workgroups (two per CU,
     // at least 4 K blocks each), fp32 partials in the split-K workspace, then their sum. A sweep of
@@ -748,7 +749,7 @@ MvPlan plan_mv(int fmt, int64_t N, int64_t K, int64_t NT, int64_t KB, int64_t M,
         // blocks per CU slower: 1500 x 4096 at 1000 (8 against 7 in two groups) 32.7 -> 34.6, 2000 x 2048 at
         // 128 (8 against 4) 17.2 -> 19.3; with two such workgroups on a CU too: 3000 x 8192 at 300 38.9 ->
         // 61.5. (g128s 32-row tiles of larger matrices keep their weights two blocks ahead instead.)
-        if (S > 1 && p.ntw == 2 && p.mb >= 2 && !(p.mb == 2 && dtile)) {
+        if (S > 1 && p.ntw == 2 && p.mb >= 2 && !(p.mb == 2 && (dtile || ed > 0))) {
             const int kg = p.mb == 8 ? 2 : 4;
             const int64_t g = es >= 1 ? S : std::min<int64_t>(KB / 4, (int64_t) cus / p.wgs * kg), planes = (g + kg - 1) / kg;
             const int64_t one = (S * p.wgs + cus - 1) / cus * ((KB + S - 1) / S), grp = g > 1 ? kg * ((KB + g - 1) / g) : KB * kg;
@@ -769,7 +770,6 @@ MvPlan plan_mv(int fmt, int64_t N, int64_t K, int64_t NT, int64_t KB, int64_t M,
     // workgroup leaves the memory idle there): 16-row tiles, and g128s 32-row tiles of larger
     // matrices (57344 x 8192 at 17-32 rows 81-84 -> 74-80 us, 24576 x 4096 24.1-25.3 -> 22.5-24.0;
     // the per-32 formats and matrices below 1e8 weights measured 1-7 % slower there)
-    const int ed = env_int("ONPU_GEMM_DEEP", -1);
     p.deep = p.ntw == 2 && p.mb <= 2 && (ed >= 0 ? ed != 0 : dtile && p.S * p.wgs <= 2 * (int64_t) cus);
     return p;
 }

@@ -166,6 +166,20 @@ def test_mv_plan_groups():
     assert (o[3], o[5], L.onpu_plan_mv_groups(2, 4096, 14336, 96)) == (16, 32, 2)
 
 
+def test_mv_plan_forced_depth(monkeypatch):
+    """ONPU_GEMM_DEEP = 1 keeps the weights of 16- and 32-row tiles two blocks ahead also where the
+    default is several K ranges per workgroup; 0 leaves those as they are"""
+    L = _lib.lib()
+    o = (C.c_int64 * 7)()
+    for fmt, N, K, M in ((0, 24576, 4096, 32), (2, 16000, 4096, 24), (3, 16000, 4096, 30)):
+        for ed, deep in ((None, 0), ("0", 0), ("1", 1)):
+            if ed is not None:
+                monkeypatch.setenv("ONPU_GEMM_DEEP", ed)
+            L.onpu_plan_mv(fmt, N, K, M, o)
+            assert o[1] == 2 and o[6] == deep and L.onpu_plan_mv_groups(fmt, N, K, M) == (1 if deep else 4), (fmt, ed, tuple(o))
+            monkeypatch.delenv("ONPU_GEMM_DEEP", raising=False)
+
+
 @pytest.mark.parametrize("fmt", [0, 1, 2, 3])
 def test_argmax_epilogue_plans_sum_like_the_store(fmt):
     """the argmax epilogue's GEMV plan (onpu_dense_argmax_dev) and the plain store's (the no-alloc
