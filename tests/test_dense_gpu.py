@@ -232,33 +232,44 @@ def test_gemm_split_k(gpu, fmt, M, N, K, mb, monkeypatch):
     check_f32_out(yf, orc.qmm(fmt, st, N, K, xb[rows], bf16w=True), what=f"split-K fmt {fmt} fp32 rows")
 
 
+# (M, N, K, forced ranges or 0, K groups per workgroup, planes of partials). 32-, 64- and 128-row tiles;
+# ranges that do not divide the groups, so that groups of the last or only plane have no K block (6, 3
+# and 7 ranges over 4 groups, 3 over 2); a last range shorter than the others; odd N; two row tiles
+K_GROUPS = [(24, 16000, 1536, 8, 4, 2), (24, 25000, 1152, 4, 4, 1), (31, 26000, 1024, 4, 4, 1),
+            (40, 14001, 1792, 8, 4, 2), (64, 25000, 1024, 4, 4, 1), (33, 16000, 4096, 0, 4, 2),
+            (96, 14300, 1152, 3, 2, 2), (96, 4096, 3584, 16, 2, 7), (70, 12345, 2048, 0, 2, 2),
+            (150, 9000, 1152, 2, 2, 1), (200, 4096, 4096, 0, 2, 4)]
+
+
 @pytest.mark.parametrize("fmt", FMTS)
-@pytest.mark.parametrize("M,N,K,S", [(24, 24576, 1024, 2), (30, 14300, 2048, 4), (40, 14000, 2048, 3), (64, 24576, 1024, 2),
-                                     (70, 12345, 1024, 2), (96, 4096, 1920, 3), (150, 9000, 1152, 2)])
-def test_gemm_k_groups(gpu, fmt, M, N, K, S, monkeypatch):
-    """GEMMs whose workgroups take several K ranges (2 or 4 groups of 4 waves), forced to S ranges: fewer
-    ranges than groups, one plane stored as Y and several, a last range shorter than the others, odd N:
-    a column slice and three rows against the oracle, and the unsplit kernel to fp32 summation order"""
+@pytest.mark.parametrize("M,N,K,S,groups,planes", K_GROUPS)
+def test_gemm_k_groups(gpu, fmt, M, N, K, S, groups, planes, monkeypatch):
+    """GEMMs whose workgroups take several K ranges (2 or 4 groups of 4 waves): fp32 and bf16 results of
+    a column slice and three rows against the oracle, a second call bit for bit, and the unsplit kernel
+    to fp32 summation order; the plan is asserted, so that a case cannot fall back to single groups"""
+    import ctypes as C
     import torch
+    from opennpu_amd import _lib
     from opennpu_amd.device import QMatrix
     if fmt != orc.FMT_G128S:
-        K -= 32
+        K -= 32                                       # a K tail inside the last 128-wide block
+    if S:
+        monkeypatch.setenv("ONPU_GEMM_SPLIT", str(S))
+    o, L = (C.c_int64 * 7)(), _lib.lib()
+    L.onpu_plan_mv(fmt, N, K, M, o)
+    g = L.onpu_plan_mv_groups(fmt, N, K, M)
+    assert (g, -(-o[3] // g)) == (groups, planes), (g, tuple(o))
     st, xb = syn.weights(fmt, N, K, 61), syn.activations(M, K, 62)
     q = QMatrix(N, K, fmt, st)
     try:
         x = to_torch_bf16(xb).reshape(M, K)
-        yd = q.mv(x, f32=True)
-        monkeypatch.setenv("ONPU_GEMM_SPLIT", str(S))
-        ys = q.mv(x, f32=True)
-        yb = q.mv(x)
+        ys, y2, yb = q.mv(x, f32=True), q.mv(x, f32=True), q.mv(x)
         monkeypatch.setenv("ONPU_GEMM_SPLIT", "1")
         y1 = q.mv(x, f32=True)
-        monkeypatch.delenv("ONPU_GEMM_SPLIT")
         torch.cuda.synchronize()
-        for y in (yd, ys):
-            # sums of K products in another order: 1e-5 of the largest, as test_gemm_split_k
-            assert ((y - y1).abs().max() / y1.abs().max()).item() <= 1e-5
-        assert torch.equal(yb, ys.to(torch.bfloat16))
+        # sums of K products in another order: 1e-5 of the largest, as test_gemm_split_k
+        assert ((ys - y1).abs().max() / y1.abs().max()).item() <= 1e-5
+        assert torch.equal(y2, ys) and torch.equal(yb, ys.to(torch.bfloat16))
         rows = [0, M // 2, M - 1]
         yc, yr = from_torch(ys[:, N - 200:]), from_torch(ys[rows])
     finally:

@@ -328,11 +328,17 @@ def test_ffn_run_reports_a_timed_out_wait(L, monkeypatch):
         L.onpu_ffn_free(f)
 
 
-@pytest.mark.parametrize("N,K,M", [(40, 128, 1), (8192, 256, 8), (8200, 256, 8), (64, 8192, 8), (64, 8320, 8),
-                                   (1000, 4096, 96)])
-def test_dense_mv_pinned_range(gpu, N, K, M):
-    """onpu_dense_mv with x and y through pinned memory, up to 256 KiB each, and past it through the
-    device staging: two inputs in turn, and again after onpu_release_scratch"""
+@pytest.mark.parametrize("N,K,M,S", [(40, 128, 1, 0), (8192, 256, 8, 0), (8200, 256, 8, 0), (64, 8192, 8, 0),
+                                     (64, 8320, 8, 0), (1000, 4096, 96, 0),
+                                     # GEMM tiles into pinned memory, and past 128 rows not
+                                     (500, 512, 96, 0), (512, 512, 128, 0), (333, 512, 100, 0), (500, 384, 129, 0),
+                                     (500, 640, 96, 2), (333, 640, 65, 5)])
+def test_dense_mv_pinned_range(gpu, N, K, M, S, monkeypatch):
+    """onpu_dense_mv with x and y through pinned memory, up to 128 rows and 256 KiB each, and past it
+    through the device staging: the GEMV, the GEMM's tiles and (S ranges of K) the sum of its partials
+    write y; two inputs in turn, and again after onpu_release_scratch"""
+    if S:
+        monkeypatch.setenv("ONPU_GEMM_SPLIT", str(S))
     import ctypes as C
     from opennpu_amd import synthetic as syn
     from opennpu_amd.device import QMatrix

@@ -145,12 +145,39 @@ def test_moe_few_rows_items(gpu, fmt, H, I):
     check_moe(y, fmt, gu, dn, E, H, I, xb, rid, rw, grouped=True, what=f"moe few rows fmt {fmt}")
 
 
+@pytest.mark.parametrize("fmt,H,I", [(orc.FMT_G128S, 2048, 768), (orc.FMT_Q4NX, 2080, 800)])
+def test_moe_few_rows_large_bank(gpu, fmt, H, I):
+    """few rows per expert in a bank above 96 MiB, whose weights are loaded non-temporally (128 experts;
+    q4nx with K tails): 24 tokens over all experts against the oracle, and 24 over the first 28 bit for
+    bit what a bank of those 28 alone gives (64 or 82 MB, plain loads)"""
+    import torch
+    E, E1, T = 128, 28, 24
+    gu, dn = _experts(fmt, E, H, I, 7000)
+    xb = syn.activations(T, H, 6)
+    x = to_torch_bf16(xb).reshape(T, H)
+    mib = (sum(map(len, gu)) + sum(map(len, dn))) / 2 ** 20
+    assert mib > 96 and mib * E1 / E < 90
+    f, f1 = _ffn(fmt, E, H, I, gu, dn), _ffn(fmt, E1, H, I, gu[:E1], dn[:E1])
+    try:
+        rid, rw = orc.route(syn.logits(T, E, 11), 8)                        # 1.5 rows per expert
+        y = from_torch(f.ffn(x, torch.from_numpy(rid).cuda(), torch.from_numpy(rw).cuda()))
+        r1, w1 = (torch.from_numpy(a).cuda() for a in orc.route(syn.logits(T, E1, 12), 4))
+        ya, yb = f.ffn(x, r1, w1), f1.ffn(x, r1, w1)
+        torch.cuda.synchronize()
+        assert torch.equal(ya, yb)
+    finally:
+        f.free()
+        f1.free()
+    check_moe(y, fmt, gu, dn, E, H, I, xb, rid, rw, grouped=True, what=f"moe few rows, large bank, fmt {fmt}")
+
+
 @pytest.mark.parametrize("fmt", [orc.FMT_Q4S, orc.FMT_Q4NX])
 def test_moe_grouped_k_tail(gpu, fmt):
     """grouped products whose K is not a multiple of 128 (H = 288 for gate+up, I = 160 for down):
-    the last K block of each reads zeros past K (the grouped GEMM's tail variant)."""
+    the last K block of each reads zeros past K (the grouped GEMM's tail variant; 25 rows per expert,
+    past the 12 up to which so small a bank runs the kernel of few rows)."""
     import torch
-    E, H, I, k, T = 8, 288, 160, 2, 40
+    E, H, I, k, T = 8, 288, 160, 2, 100
     gu, dn = _experts(fmt, E, H, I, 5000)
     xb = syn.activations(T, H, 7)
     rid, rw = orc.route(syn.logits(T, E, 8), k)
