@@ -742,18 +742,27 @@ MvPlan plan_mv(int fmt, int64_t N, int64_t K, int64_t NT, int64_t KB, int64_t M,
         int64_t S = es >= 1 ? es : std::min<int64_t>(KB / 4, 2 * (int64_t) cus / p.wgs);
         // K groups of one workgroup (k_qgemm's KG, one workgroup per CU): the partials are planes, not
         // ranges, or go with their sum launch. Taken where no CU gets more K blocks than with single
-        // groups (for up to 64 rows a fifth more, as the partials weigh more). us per call, one group ->
-        // KG, 3 matrices in turn: 24576 x 4096 at 32 rows q4nx 24.2 -> 20.5, 4096 x 14336 at 24 / 96 14.3 /
-        // 30.5 -> 13.4 / 28.5, 14336 x 4096 at 30 / 48 / 100 15.9 / 20.2 / 32.2 -> 14.8 / 18.3 / 30.6, 4096 x
-        // 4096 at 200 28.6 -> 25.9, 12345 x 2048 at 70 26.6 -> 21.8, 9000 x 1056 at 150 23.7 -> 18.6. With more
-        // blocks per CU slower: 1500 x 4096 at 1000 (8 against 7 in two groups) 32.7 -> 34.6, 2000 x 2048 at
-        // 128 (8 against 4) 17.2 -> 19.3; with two such workgroups on a CU too: 3000 x 8192 at 300 38.9 ->
-        // 61.5. (g128s 32-row tiles of larger matrices keep their weights two blocks ahead instead.)
+        // groups (a sixth more with tiles of 32 rows, a fifth with 64, whose partials weigh more). us per
+        // call, one group -> KG, 3 matrices in turn: 24576 x 4096 at 32 rows q4nx 24.2 -> 20.5, 4096 x 14336
+        // at 24 / 96 14.3 / 30.5 -> 13.4 / 28.5, 14336 x 4096 at 30 / 48 / 100 15.9 / 20.2 / 32.2 -> 14.8 /
+        // 18.3 / 30.6, 4096 x 4096 at 200 28.6 -> 25.9, 12345 x 2048 at 70 26.6 -> 21.8, 9000 x 1056 at 150
+        // 23.7 -> 18.6. With more blocks per CU slower: 1500 x 4096 at 1000 (8 against 7 in two groups) 32.7
+        // -> 34.6, 2291 x 4352 at 188 (10 against 5) 25.2 -> 26.5, 11136 x 9216 q4nx at 21 (36 against 30)
+        // 24.9 -> 26.0; with two such workgroups on a CU too: 3000 x 8192 at 300 38.9 -> 61.5.
+        // The two groups of a 128-row tile step together, where two workgroups of a CU do not: ~0.2 us per K
+        // block, against the fixed gain of the planes and the launch. So up to 60 blocks per CU with one
+        // plane (no sum), 28 with more; past that the mean over 250 shapes turns: one plane, 4224 x 11136 at
+        // 893 rows (88 blocks) 118.4 -> 122.9, 11200 x 11136 at 144 (88) 106.6 -> 118.3, 8260 x 16256 at 259
+        // (128) 148.4 -> 170.7; two, 6957 x 13184 at 194 (52) 75.8 -> 80.8, 13376 x 12160 at 116 (48) 67.2 ->
+        // 72.4. Tiles of 32 and 64 rows gain at any length (31552 x 7424 at 48, 60 blocks: 59.3 -> 52.5).
+        // (g128s 32-row tiles of larger matrices keep their weights two blocks ahead instead.)
         if (S > 1 && p.ntw == 2 && p.mb >= 2 && !(p.mb == 2 && (dtile || ed > 0))) {
             const int kg = p.mb == 8 ? 2 : 4;
             const int64_t g = es >= 1 ? S : std::min<int64_t>(KB / 4, (int64_t) cus / p.wgs * kg), planes = (g + kg - 1) / kg;
-            const int64_t one = (S * p.wgs + cus - 1) / cus * ((KB + S - 1) / S), grp = g > 1 ? kg * ((KB + g - 1) / g) : KB * kg;
-            if (g > 1 && planes * p.wgs <= cus && (p.mb == 8 ? grp <= one : 5 * grp <= 6 * one)) {
+            const int64_t kb1 = (KB + S - 1) / S, one = ((KB + kb1 - 1) / kb1 * p.wgs + cus - 1) / cus * kb1;
+            const int64_t grp = g > 1 ? kg * ((KB + g - 1) / g) : KB * kg;
+            if (g > 1 && planes * p.wgs <= cus &&
+                (p.mb == 8 ? grp <= one && grp <= (planes == 1 ? 60 : 28) : p.mb == 4 ? 5 * grp <= 6 * one : 6 * grp <= 7 * one)) {
                 p.kg = kg;
                 S = g;
             }

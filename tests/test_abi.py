@@ -166,6 +166,19 @@ def test_mv_plan_groups():
     assert (o[3], o[5], L.onpu_plan_mv_groups(2, 4096, 14336, 96)) == (16, 32, 2)
 
 
+@pytest.mark.parametrize("fmt,N,K,M,S", [
+    (2, 11200, 11136, 144, 2), (3, 3200, 15616, 830, 2), (2, 8260, 16256, 259, 2),       # one plane, over 60 blocks per CU
+    (2, 6957, 13184, 194, 4), (2, 13376, 12160, 116, 4), (1, 6656, 12160, 139, 4),       # two planes, over 28
+    (3, 2291, 4352, 188, 7), (0, 11136, 9216, 21, 5), (2, 1500, 4096, 1000, 5)])         # more blocks per CU
+def test_mv_plan_single_groups(fmt, N, K, M, S):
+    """GEMMs that several K groups per workgroup slow down (2-15 % measured) keep single groups, in S
+    ranges: long K in 128-row tiles, and shapes whose busiest CU would get more K blocks"""
+    L = _lib.lib()
+    o = (C.c_int64 * 7)()
+    L.onpu_plan_mv(fmt, N, K, M, o)
+    assert (o[0], o[3], L.onpu_plan_mv_groups(fmt, N, K, M)) == (1, S, 1), tuple(o)
+
+
 def test_mv_plan_forced_depth(monkeypatch):
     """ONPU_GEMM_DEEP = 1 keeps the weights of 16- and 32-row tiles two blocks ahead also where the
     default is several K ranges per workgroup; 0 leaves those as they are"""

@@ -233,9 +233,9 @@ def test_gemm_split_k(gpu, fmt, M, N, K, mb, monkeypatch):
 
 
 # (M, N, K, forced ranges or 0, K groups per workgroup, planes of partials). 32-, 64- and 128-row tiles;
-# ranges that do not divide the groups, so that groups of the last or only plane have no K block (6, 3
-# and 7 ranges over 4 groups, 3 over 2); a last range shorter than the others; odd N; two row tiles
-K_GROUPS = [(24, 16000, 1536, 8, 4, 2), (24, 25000, 1152, 4, 4, 1), (31, 26000, 1024, 4, 4, 1),
+# ranges that do not divide the groups, so that groups of the last plane have no K block (7 ranges over
+# 4 groups, 3 over 2); a last range shorter than the others; odd N; two row tiles
+K_GROUPS = [(24, 14001, 1792, 8, 4, 2), (24, 16000, 4224, 0, 4, 2), (31, 26000, 1024, 4, 4, 1),
             (40, 14001, 1792, 8, 4, 2), (64, 25000, 1024, 4, 4, 1), (33, 16000, 4096, 0, 4, 2),
             (96, 14300, 1152, 3, 2, 2), (96, 4096, 3584, 16, 2, 7), (70, 12345, 2048, 0, 2, 2),
             (150, 9000, 1152, 2, 2, 1), (200, 4096, 4096, 0, 2, 4)]
