@@ -956,18 +956,25 @@ hipError_t moe_decode_two(Ffn * f, const uint16_t * x, int64_t T, int k, const i
     return launch_qgemv(dn->fmt, EPI_SLOTSUM_, b, 1, 1, pd.nb, 0, dim3((unsigned) dn->g.NT, (unsigned) T), pd.kw, s);
 }
 
-// routed-expert FFN on device data (act 0, no biases): x bf16 [T][H], ids/w [T][k] -> y [T][Nd]
 // k_moe_few (items of 16 rows, workgroups of half the columns, no LDS) against k_moe_gemm for n routed
 // rows: up to 1.5 rows per expert, where nearly every item is one A block anyway, and further where the
-// 8-wave workgroups of gate+up leave CUs idle (us per layer, k_moe_gemm -> k_moe_few, 3 banks in turn):
-//   128 experts, H 2048, I 768, k 8 (768 workgroups): 6 / 24 tokens 44.2 / 75.0 -> 40.4 / 69.2, q4nx
-//     49.1 / 83.6 -> 44.6 / 79.3; 32 tokens (2 rows) 76.1 -> 75.7, q4nx 85.4 -> 87.0; 64 tokens 78.4 -> 79.6
+// 8-wave workgroups of gate+up leave CUs idle. us per layer, k_moe_gemm -> k_moe_few, both with moe_nt's
+// loads, banks and logits in turn, other geometries beside Qwen3-30B-A3B's (128 experts, H 2048, I 768,
+// k 8: 768 workgroups):
+//   that at 8 / 16 / 24 tokens g128s 51.8 / 66.5 / 76.0 -> 49.4 / 64.0 / 72.2, q4nx 58.1 / 75.6 / 87.6 ->
+//     56.0 / 74.1 / 82.7; 32 tokens (2 rows, plain loads) 76.1 -> 75.7, q4nx 85.4 -> 87.0; 64 tokens 78.4
+//     -> 79.6. Over 30-60 geometries with up to 1.5 rows per expert, mean ratio g128s 0.88, q4nx 0.88
+//   q4s and q4_0 (0.93) not with a K of 1024 or more and more than 96 rows, where most experts are active
+//     and fill the GPU either way: 128 experts, H 3072, I 512 at 168 rows 75.8 -> 81.8, H 1280, I 1536 at 119
+//     73.8 -> 78.0, 256 experts, H 3328, I 256 at 381 82.3 -> 91.8 (mean of 13 shapes 1.03); with H below 1024
+//     0.98 (256 experts, H 640, I 1024 at 135 50.0 -> 45.3)
 //   one per CU or fewer, to 5 rows: 32 experts, I 1024, k 4 at 40 tokens 43.1 -> 39.6, at 100 45.6 -> 57.0
 //   one per two CUs, to 12: 8 experts, H 4096, I 2048, k 2 at 10 / 40 tokens 57.9 / 59.0 -> 39.6 / 41.1,
 //     at 64 64.3 -> 66.0
-bool moe_few(int64_t n, int64_t E, int64_t I) {
+bool moe_few(int fmt, int64_t n, int64_t E, int64_t H, int64_t I) {
     const int64_t cus = device().cus > 0 ? device().cus : 256, wgs = E * ((I / 16 + 7) / 8);
-    return 2 * n <= 3 * E || (wgs <= cus && n <= 5 * E) || (2 * wgs <= cus && n <= 12 * E);
+    const bool late = (fmt == ONPU_Q4S || fmt == ONPU_Q4_0) && n > 96 && H >= 1024;
+    return (2 * n <= 3 * E && !late) || (wgs <= cus && n <= 5 * E) || (2 * wgs <= cus && n <= 12 * E);
 }
 
 // Non-temporal weight loads for a bank of more than 96 MiB, which no 256 MiB last-level cache keeps from
@@ -975,8 +982,13 @@ bool moe_few(int64_t n, int64_t E, int64_t I) {
 // (us per layer, plain -> non-temporal): 311 MB at 24 / 64 / 128 / 700 tokens 74.6 / 82.3 / 83.8 / 115.6 ->
 // 69.2 / 78.4 / 80.5 / 114.6, q4nx (377 MB) at 128 101.8 -> 91.3; at 1000 tokens (62 rows per expert, many
 // read twice) 157.3 -> 161.0. Banks of 78 and 13 MB, which stay cached: 32.0 -> 34.2, 27.1 -> 28.5.
+// The figures above are with three banks in turn. With up to six (2.5 GB) and other logits on each call, 8
+// geometries of 8-256 experts at 5-512 tokens, 0.5-12 % faster, also where few experts are active (5 tokens
+// 40.0 -> 38.6, q4nx 46.0 -> 44.5); a loop over one bank with one input, whose experts then stay cached
+// up to ~280 MB of them, is 3-18 % slower (5 tokens 36.2 -> 38.9).
 bool moe_nt(int64_t n, int64_t E, int64_t bytes) { return bytes > ((int64_t) 96 << 20) && n <= 48 * E; }
 
+// routed-expert FFN on device data (act 0, no biases): x bf16 [T][H], ids/w [T][k] -> y [T][Nd]
 hipError_t ffn_core(Ffn * f, const uint16_t * x, int64_t T, const int32_t * ids, int k, const float * w, void * y,
                     int yf32, hipStream_t s) {
     Mat4 * gu = f->gu, * dn = f->dn;
@@ -995,7 +1007,7 @@ hipError_t ffn_core(Ffn * f, const uint16_t * x, int64_t T, const int32_t * ids,
     }
     // prompts: tokens grouped per expert (one pass over each routed expert's weights per 64 rows)
     const int64_t E = gu->E;
-    const bool few = moe_few(n, E, I), nt = moe_nt(n, E, E * (gu->dstride + dn->dstride));
+    const bool few = moe_few(gu->fmt, n, E, gu->K, I), nt = moe_nt(n, E, E * (gu->dstride + dn->dstride));
     const int rows_per_item = few ? 16 : 64;      // one A block, or the grouped GEMM's 4
     const int64_t maxitems = n / rows_per_item + E;
     if ((e = f->ws[1].ensure((size_t) (E + 1) * 4)) != hipSuccess) return e;
