@@ -400,10 +400,10 @@ __global__ __launch_bounds__(MT, 2) void k_attn_mfma(AttnArgs a) {
             up = up || m[h4] != mx;
             m[h4] = mx;
             l[h4] *= al[h4];
-            const float base = mx == -__builtin_inff() ? 0.f : mx;           // -inf rows alone: p = 0; NaN: p = NaN
 #pragma unroll
             for (int t = 0; t < KT; t++) {
-                const float p = expf(sc[t][h4] - base);
+                // 0 also while the maximum is -inf; NaN, which the maximum skips, stays NaN
+                const float p = sc[t][h4] == -__builtin_inff() ? 0.f : expf(sc[t][h4] - mx);
                 l[h4] += p;
                 if (4 * h4 + quad < HG) P[(16 * t + key) * HG + 4 * h4 + quad] = p;
             }
@@ -677,9 +677,18 @@ hipError_t launch_attn_step(const float * q, int Hq, int D, const void * K, cons
     if (rs % al || hs % al || ((uintptr_t) K | (uintptr_t) V | (uintptr_t) q) % 16) return hipErrorInvalidValue;
     if (ws_bytes < attn_ws_bytes(Hq, D, Hkv, S)) return hipErrorInvalidValue;
     AttnPlan p = attn_plan(Hq, D, Hkv, S);
-    // Four passes (two at D > 128) in one workgroup cost no more than one pass, the second launch and its
-    // read of the partials: 32 / 8 heads, D = 128, 300 and 500 rows 8.2 and 9.5 us against 6.7 + 3.1, a
-    // call 13.4 -> 10.4 us from Python; D = 256, 300 rows in one workgroup 16.9 us against 13.5.
+    // One workgroup per head group, without the second launch, up to four of its passes (two at D > 128):
+    // a call issued from Python pays for the launch, and at four passes about breaks even. us per call, two
+    // launches -> one, issued from Python / replayed from a graph of 16 calls:
+    //   32 / 8 heads, D = 128: 128 rows 9.7 / 7.8 -> 7.2 / 5.3, 384 9.4 / 7.9 -> 8.4 / 8.4, 512 9.7-10.9 / 7.8 ->
+    //     9.9 / 9.9
+    //   40 / 8 (8 heads per group): 128 rows 9.9 / 8.6 -> 7.5 / 7.5, 192 10.0 / 8.6 -> 8.9 / 8.9, 256 10.0-10.8 / 8.7
+    //     -> 10.2 / 10.3
+    //   64 / 8, D = 64: 256 rows 9.8 / 7.4 -> 8.1 / 8.1; 32 / 8, D = 64: 512 rows 10.0 / 6.8 -> 7.3 / 6.7
+    //   8 / 8 and 16 / 8, D = 128: 384 rows 9.6 / 6.7 -> 7.2 / 6.1 and 9.9 / 7.0 -> 7.3 / 6.8, 512 9.5 / 6.7 -> 7.2 /
+    //     7.2 and 9.9 / 7.1 -> 8.0 / 8.0
+    //   D = 256, 16 / 2, 16 / 4 and 8 / 8: 128 rows 11.4 / 11.4, 10.0 / 8.9 and 10.1 / 6.9 -> 11.3 / 11.4, 8.1 / 8.2
+    //     and 7.4 / 5.4; 300 rows in one workgroup 16.9 against 13.5
     const int64_t one = D > 128 ? 128 : (p.HG >= 8 ? 256 : 512);
     if (kv_bf16 && S <= one) {
         p.C = (int) S;
