@@ -27,7 +27,7 @@ constexpr int AW = AT / 64;
 constexpr int AU = 4;                        // rows per lane group in flight
 constexpr int AP_MAX = 16384;                // floats of P per workgroup (64 KiB)
 constexpr int TARGET_WG = 512;
-constexpr int ATT_MAX_CH = 4096;             // chunks per kv head at most (the combine's LDS)
+constexpr int ATT_MAX_CH = 4096;             // chunks per kv head at most: 8M rows or more, past any cache
 
 struct AttnArgs {
     const float * q;

@@ -1,8 +1,11 @@
 // Weight codecs of libonpu_hip, one source for the host quantizers behind onpu_pack /
 // onpu_pack_q4k (onpu_quant.cpp) and their GPU versions behind onpu_quantize_dev /
-// onpu_transcode_q4k_dev (onpu_codec.hip), so that both write the same staging bytes.
-// Every multiply and add is rounded on its own (no contraction into fused multiply-adds), divisions
-// are IEEE fp32 and rint rounds half to even, on the host and on the GPU alike.
+// onpu_transcode_q4k_dev (onpu_codec.hip). What they share is the values: the host writes staging bytes and
+// the GPU tiles with the same codes, scales and mins. Here every multiply and add is rounded on its own (no
+// contraction into fused multiply-adds), divisions are IEEE fp32 and rint rounds half to even, on the
+// host and, where the GPU runs this source (Q4_0, groups out of the searches' range), there too; the
+// GPU's searches take their quotients by reciprocal and fuse exact products, as onpu_codec.hip derives,
+// and q4k_sub fuses one exact product.
 #pragma once
 #include "onpu_common.h"
 

@@ -32,10 +32,12 @@ __device__ __forceinline__ void load_group(const void * W, int64_t off, float (&
 // ------------------------------------------------------------------ search quantizers
 // The searches of onpu_codec.h without their divisions. VALU-bound: an IEEE division is ~10 of the ~19
 // ops a pass takes per weight; without it a q4s candidate takes 12.5 ops per weight from bf16 (16 from
-// fp32) instead of 36. Whole call, 12288 x 4096, from bf16 / fp32: q4s 882 / 870 -> 224 / 309 us, g128s
+// fp32) instead of 36. (Counters, 24576 x 4096 q4s from bf16: 14.2 VALU instructions per weight and candidate
+// with all that is around the two passes, one per 2.7 cycles of a SIMD; waves wait for memory in 5 % of
+// their cycles and for their turn to issue in 64 %; q4nx 3 and 62 %.) Whole call, 12288 x 4096, from bf16 / fp32: q4s 882 / 870 -> 224 / 309 us, g128s
 // 889 / 905 -> 247 / 338, q4nx 897 / 899 -> 361 / 396; Q4_0, which has no search, 200 / 222 -> 40 / 58
-// (no staging); q4s 24576 x 4096 from bf16 1728 -> 439. Every value that reaches a code, a scale or a comparison is the same fp32
-// number as there:
+// (no staging); q4s 24576 x 4096 from bf16 1728 -> 439. Every value that reaches a code, a scale or a
+// comparison is the same fp32 number as there:
 //   - v x, l x (4-bit integer times bf16), v v, l sc, v d (d, sc are bf16 values) are exact products, so
 //     one fma rounds as the multiply and the add do;
 //   - a quotient only reaches rint(RN(x / d)). With r ~ 1 / d within 2^-23.9 of it relative,

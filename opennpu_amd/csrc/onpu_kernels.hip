@@ -238,8 +238,8 @@ __global__ __launch_bounds__(1024) void k_gemv_i8(const int8_t * __restrict__ W,
     const int64_t row0 = ((int64_t) blockIdx.x * (blockDim.x >> (6 + lks)) + gl) * GI8_R;
     const int nr = N - row0 >= GI8_R ? GI8_R : (N > row0 ? (int) (N - row0) : 0);
     const int k0 = (wave - gl * ks) * Kw, k1 = k0 + Kw < K ? k0 + Kw : K;
-    // Buffer loads without branches: x past the slice reads as zero, W past the rows too (and past the
-    // slice inside them bytes that meet those zeros)
+    // Buffer loads without branches (the range check counts the scalar offset): x past the slice reads as
+    // zero, W past the rows too (and past the slice inside them bytes that meet those zeros)
     const __amdgpu_buffer_rsrc_t xr = __builtin_amdgcn_make_buffer_rsrc((void *) x, (short) 0, k1 * 4, 0x00020000);
     const __amdgpu_buffer_rsrc_t wr =
         __builtin_amdgcn_make_buffer_rsrc((void *) (W + (nr ? row0 : 0) * K), (short) 0, nr * K, 0x00020000);
@@ -791,7 +791,8 @@ hipError_t launch_moe_act(const float * h, int64_t rows, int64_t Ng, const int32
 hipError_t launch_gemv_i8(const int8_t * W, const float * sc, int64_t N, int64_t K, const float * x, float * y,
                           hipStream_t s) {
     if (N <= 0 || K <= 0) return hipSuccess;
-    if (K % 16 || K * 4 > 128 * 1024 || ((uintptr_t) W | (uintptr_t) x) % 16) return hipErrorInvalidValue;
+    // K <= 32768 is the documented limit; the 32-bit buffer offsets (4 K, and 4 rows of K bytes) hold far more
+    if (K % 16 || K > 32768 || ((uintptr_t) W | (uintptr_t) x) % 16) return hipErrorInvalidValue;
     const int64_t ng = (N + GI8_R - 1) / GI8_R;
     // K slices until there are 8 waves per CU or a slice is 1024 long (one batch of 4 loads per row):
     // with few rows the waves in flight are what brings the bytes in (512 x 16384, 16 slices: 11.5 ->

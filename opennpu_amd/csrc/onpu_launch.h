@@ -227,9 +227,9 @@ int chain_occupancy(int fmt, int ring, size_t lds);
 // layout (dst, dstride apart); packed row r becomes staging row rowmap[r] (r when rowmap is null)
 hipError_t launch_npu_stage(int fmt, const uint8_t * src, int64_t sstride, const NpuGeom & g, const int32_t * rowmap,
                             int64_t N, int64_t K, uint8_t * dst, int64_t dstride, int64_t E, hipStream_t s);
-// p[0, n) = 0 by a kernel on stream s (a graph node under capture, unlike a memset)
 // *word = tag (host memory the GPU sees), after all earlier work on s
 hipError_t launch_host_word(uint32_t * word, uint32_t tag, hipStream_t s);
+// p[0, n) = 0 by a kernel on stream s (a graph node under capture, unlike a memset)
 hipError_t launch_zero_i32(int32_t * p, int64_t n, hipStream_t s);
 // y[t] = sum_j w[t][j] o[inv[t k + j]] (o bf16 rows, fp32 sum)
 hipError_t launch_moe_combine(const uint16_t * o, const int32_t * inv, const float * w, int64_t T, int k, int64_t N,
@@ -259,7 +259,7 @@ hipError_t launch_quantize(int fmt, const void * W, int64_t ldw, int wbf16, int6
                            uint8_t * out, int64_t ostride, hipStream_t s);
 hipError_t launch_q4k(const uint8_t * blocks, int64_t ld, int64_t bstride, int64_t N, int64_t K, int64_t ne,
                       uint8_t * out, int64_t ostride, hipStream_t s);
-// int8 GEMV y = s * (W x) for int8 W [N][K] rows (K a multiple of 16, K * 4 bytes of x in LDS)
+// int8 GEMV y = s * (W x) for int8 W [N][K] rows (K a multiple of 16, at most 32768)
 hipError_t launch_gemv_i8(const int8_t * W, const float * sc, int64_t N, int64_t K, const float * x, float * y,
                           hipStream_t s);
 // Gated DeltaNet decode step (onpu_attn.hip): workspace of the conv outputs, and the two launches

@@ -34,6 +34,27 @@ def test_gemv_i8_dev(gpu, N, K):
     assert err <= 1e-5, err
 
 
+@pytest.mark.parametrize("N,K", [(1, 16), (1, 272), (3, 528), (6, 2320), (5, 32752)])
+def test_gemv_i8_dev_reads_only_its_operands(gpu, N, K):
+    """W and x in the middle of larger tensors, x between NaNs: the loads past a slice's and a row's end
+    give zeros and not the neighbours"""
+    import torch
+    rng = np.random.default_rng(K)
+    pad = 16384
+    W = rng.integers(-128, 128, N * K + 2 * pad).astype(np.int8)
+    x = np.full(K + 2 * pad, np.nan, np.float32)
+    x[pad:pad + K] = rng.standard_normal(K)
+    s = rng.uniform(1e-3, 2e-2, N).astype(np.float32)
+    Wd, xd, sd = (torch.from_numpy(a).cuda() for a in (W, x, s))
+    y = torch.full((N + 64,), 7.0, dtype=torch.float32, device="cuda")
+    print(f"gemv_i8_dev inside larger tensors N={N} K={K}", flush=True)
+    assert gpu.onpu_gemv_i8_dev(Wd.data_ptr() + pad, sd.data_ptr(), N, K, xd.data_ptr() + 4 * pad, y.data_ptr(), None) == 0
+    torch.cuda.synchronize()
+    got, ref = y.cpu().numpy(), orc.gemv_i8(W[pad:pad + N * K].reshape(N, K), s, x[pad:pad + K])
+    assert np.abs(got[:N] - ref).max() <= 1e-5 * np.abs(ref).max()
+    assert (got[N:] == 7.0).all()
+
+
 def test_gemv_i8_dev_argument_errors(gpu):
     import torch
     L = gpu
@@ -41,5 +62,5 @@ def test_gemv_i8_dev_argument_errors(gpu):
     v = torch.zeros((64,), dtype=torch.float32, device="cuda")
     P = lambda t: C.c_void_p(t.data_ptr())
     assert L.onpu_gemv_i8_dev(P(W), P(v), 4, 40, P(v), P(v), None) == -1           # K % 16
-    assert L.onpu_gemv_i8_dev(P(W), P(v), 4, 65536, P(v), P(v), None) == -1        # x past the LDS copy
+    assert L.onpu_gemv_i8_dev(P(W), P(v), 4, 65536, P(v), P(v), None) == -1        # past the documented K
     assert b"onpu_gemv_i8_dev" in L.onpu_last_error()
