@@ -123,7 +123,11 @@ DBuf g_hws[12];
 // place; and a word that a last kernel sets to the call's tag, so that the host sees the end of the
 // call without a stream synchronisation. A 4096 x 4096 q4nx product of one row through two pageable
 // copies and a synchronisation took 35 us, 26 of them outside its kernels; so 21 (8192 x 8192 at 8 rows
-// 66 -> 47). Coherent memory: a kernel's stores pass the caches, and are out when it has completed.
+// 66 -> 47). Coherent memory: a kernel's stores pass the caches, and are out when it has completed. The gain
+// is the same 16-22 us at every size, so the limits are not where it ends: 256 KiB each bounds what stays pinned,
+// and more than 128 rows may run the stream-K GEMM, whose wait flag the other path reads (us per call,
+// staged -> pinned: 512 x 512 at 1 / 24 / 64 / 128 rows 30.0 / 38.3 / 47.2 / 59.1 -> 14.0 / 19.8 / 29.1 / 40.1, 4096 x
+// 4096 at 16 54.4 -> 36.1, 682 x 640 at 96 59.6 -> 40.7, 512 x 65536 at 1 96.9 -> 78.9; 78 calls in all, none slower).
 constexpr size_t HP_BYTES = 256 << 10;       // x and y up to this size each
 struct HostPin {
     uint8_t * p = nullptr;
@@ -751,7 +755,7 @@ MvPlan plan_mv(int fmt, int64_t N, int64_t K, int64_t NT, int64_t KB, int64_t M,
         // 24.9 -> 26.0; with two such workgroups on a CU too: 3000 x 8192 at 300 38.9 -> 61.5.
         // The two groups of a 128-row tile step together, where two workgroups of a CU do not: ~0.2 us per K
         // block, against the fixed gain of the planes and the launch. So up to 60 blocks per CU with one
-        // plane (no sum), 28 with more; past that the mean over 250 shapes turns: one plane, 4224 x 11136 at
+        // plane (no sum), 28 with more; past that the mean over 200 shapes turns: one plane, 4224 x 11136 at
         // 893 rows (88 blocks) 118.4 -> 122.9, 11200 x 11136 at 144 (88) 106.6 -> 118.3, 8260 x 16256 at 259
         // (128) 148.4 -> 170.7; two, 6957 x 13184 at 194 (52) 75.8 -> 80.8, 13376 x 12160 at 116 (48) 67.2 ->
         // 72.4. Tiles of 32 and 64 rows gain at any length (31552 x 7424 at 48, 60 blocks: 59.3 -> 52.5).

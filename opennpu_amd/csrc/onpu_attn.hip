@@ -229,7 +229,7 @@ __global__ __launch_bounds__(AT) void k_attn_part(AttnArgs a) {
 // A wave takes 16 KT rows at a time. Bound by VALU work and latency at short context, by HBM at long.
 // (The kernel above, which bf16 took too, spent its time in four barriers, P in LDS per workgroup and a
 // DPP sum per row and head. Both launches, us per call, Hq / Hkv / D at S rows: 32 / 8 / 128 at 8192
-// 17.8 -> 12.9, at 65536 53.6 -> 52.0 (5.2 TB/s); 32 / 4 / 128 at 16384 36.8 -> 14.8; 64 / 8 / 64 at 65536
+// 17.8 -> 12.0, at 65536 53.6 -> 52.0 (5.2 TB/s); 32 / 4 / 128 at 16384 36.8 -> 14.8; 64 / 8 / 64 at 65536
 // 61.7 -> 30.9; 16 / 2 / 256 at 16384 44.6 -> 22.2; 40 / 8 / 128 at 65536 93.6 -> 53.1. Error against 64 bits at
 // those layouts 1.6-2.2e-7 -> 1.6-1.85e-7.) A row of an
 // MFMA's A operand is one of three bf16 parts of one of 4 heads' q (row 4 h + part): q cut at its bits,
